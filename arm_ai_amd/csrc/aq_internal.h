@@ -451,7 +451,7 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Wave-uniform max / min over all 64 lanes (all lanes active): max within
+// Wave-uniform max over all 64 lanes (all lanes active): max within
 // each row of 16 lanes by DPP, then across the four rows by readlane.
 __device__ __forceinline__ float wave_max_f(float v) {
     v = fmaxf(v, dpp_f<DPP_QUAD_XOR1>(v));
@@ -459,14 +459,6 @@ __device__ __forceinline__ float wave_max_f(float v) {
     v = fmaxf(v, dpp_f<DPP_HALF_MIRROR>(v));
     v = fmaxf(v, dpp_f<DPP_ROW_MIRROR>(v));
     return fmaxf(fmaxf(readlane_f(v, 0), readlane_f(v, 16)), fmaxf(readlane_f(v, 32), readlane_f(v, 48)));
-}
-__device__ __forceinline__ int wave_min_i(int v) {
-    v = min(v, dpp_i<DPP_QUAD_XOR1>(v));
-    v = min(v, dpp_i<DPP_QUAD_XOR2>(v));
-    v = min(v, dpp_i<DPP_HALF_MIRROR>(v));
-    v = min(v, dpp_i<DPP_ROW_MIRROR>(v));
-    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
 // One Q8_K block (candle-core 0.8.4 BlockQ8K::from_float) quantised by one
@@ -477,7 +469,8 @@ __device__ __forceinline__ int wave_min_i(int v) {
 // so max is the FIRST element of largest |x| (NaN never wins); then
 // iscale = -128/max, q = min(round(iscale*x), 127) with ties away from zero,
 // d = 1/iscale; an all-zero block gives d = 0, q = 0.  Here: amax = max |x|
-// over the wave, then the smallest index attaining it, then that element.
+// over the wave, then the first lane attaining it (a ballot), then its first
+// element that does.
 // IEEE division (the library is built without fast-math) keeps it bit-exact.
 __device__ __forceinline__ uint32_t q8k_block_wave(const float v[4], int lane, int *bsum, float *d) {
     float ax[4];
@@ -490,14 +483,15 @@ __device__ __forceinline__ uint32_t q8k_block_wave(const float v[4], int lane, i
     int q[4] = {0, 0, 0, 0};
     float dd = 0.0f;
     if (am != 0.0f) {  // uniform
-        int li = 1 << 30;
+        // the first lane that holds the maximum, and its first element that is it
+        float mine = v[3];
+        bool has = ax[3] == am;
 #pragma unroll
-        for (int i = 3; i >= 0; i--)
-            if (ax[i] == am) li = 4 * lane + i;
-        const int idx = wave_min_i(li);
-        const int c = idx & 3;
-        const float mine = c == 0 ? v[0] : c == 1 ? v[1] : c == 2 ? v[2] : v[3];
-        const float mx = readlane_f(mine, idx >> 2);
+        for (int i = 2; i >= 0; i--) {
+            if (ax[i] == am) mine = v[i];
+            has |= ax[i] == am;
+        }
+        const float mx = readlane_f(mine, __builtin_ctzll(__ballot(has)));
         const float iscale = -128.0f / mx;
 #pragma unroll
         for (int i = 0; i < 4; i++) q[i] = sat_i8(fminf(roundf(iscale * v[i]), 127.0f));

@@ -12,18 +12,16 @@ namespace aq {
 
 // One wavefront per 256-element block, lane l holding elements 4l..4l+3
 // (q8k_block_wave, the fused prologues' code): four blocks per 256-thread
-// workgroup.  The block's row and index within the row are wave-uniform
-// (scalar arithmetic).
+// workgroup.
 template <bool VEC>
 __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float *__restrict__ x, int64_t nblocks,
-                                                           int64_t k, ActPlanes a) {
+                                                           ActPlanes a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t bi = (int64_t)blockIdx.x * 4 + wave;
     if (bi >= nblocks) return;  // uniform over the wavefront
-    const int64_t nb = k / QK_K;
-    const int64_t row = bi / nb, sb = bi - row * nb;
-    const int64_t e0 = row * k + sb * QK_K + 4 * lane;
+    // (blocks, bsums and d lie one after the other over the rows: no row index)
+    const int64_t e0 = bi * QK_K + 4 * lane;
     float v[4];
     if (VEC) {
         const float4 t = *(const float4 *)(x + e0);
@@ -38,21 +36,20 @@ __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float *__restri
     int bsum;
     float d;
     const uint32_t packed = q8k_block_wave(v, lane, &bsum, &d);
-    store_q8k_block64(a, row, k, sb, lane, packed, bsum, d);
+    store_q8k_block64(a, 0, 0, bi, lane, packed, bsum, d);
 }
 
 // Eight lanes per 32-element block, 32 blocks per workgroup.
 template <bool VEC>
 __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restrict__ x, int64_t nblocks,
-                                                            int64_t k, ActPlanes a) {
+                                                            ActPlanes a) {
     const int64_t gb = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
     const int sub = threadIdx.x & 7;
     const bool valid = gb < nblocks;
-    const int64_t nb = k / QK8_0;
-    const int64_t row = valid ? gb / nb : 0, b = valid ? gb - row * nb : 0;
+    const int64_t e0 = gb * QK8_0 + 4 * sub;  // (blocks lie one after the other over the rows)
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (valid) {
-        const float *xb = x + row * k + b * QK8_0 + 4 * sub;
+        const float *xb = x + e0;
         if (VEC) {
             const float4 t = *(const float4 *)xb;
             v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
@@ -63,10 +60,10 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restr
     uint16_t h;
     const uint32_t packed = q8_0_block_8lanes(v, &h);
     if (!valid) return;
-    *(uint32_t *)(a.qs + row * k + b * QK8_0 + 4 * sub) = packed;
+    *(uint32_t *)(a.qs + e0) = packed;
     if (sub == 0) {
-        a.d16[row * nb + b] = h;
-        a.d[row * nb + b] = f16_bits_to_f32(h);
+        a.d16[gb] = h;
+        a.d[gb] = f16_bits_to_f32(h);
     }
 }
 
@@ -77,9 +74,9 @@ hipError_t launch_quantize_q8k(const float *x, int64_t m, int64_t k, ActPlanes a
     const int64_t grid = (nblocks + 3) / 4;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     if (((uintptr_t)x & 15) == 0)
-        quantize_q8k_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
+        quantize_q8k_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
     else
-        quantize_q8k_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
+        quantize_q8k_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
     return hipGetLastError();
 }
 
@@ -90,9 +87,9 @@ hipError_t launch_quantize_q8_0(const float *x, int64_t m, int64_t k, ActPlanes 
     const int64_t grid = (nblocks + 31) / 32;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     if (((uintptr_t)x & 15) == 0)
-        quantize_q8_0_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
+        quantize_q8_0_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
     else
-        quantize_q8_0_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
+        quantize_q8_0_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
     return hipGetLastError();
 }
 
