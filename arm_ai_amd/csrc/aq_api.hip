@@ -234,7 +234,7 @@ int run_matmul(aq_ctx *ctx, const aq_qweight *w, const float *d_x, int64_t m, fl
     hipError_t e;
     if (use_gemm(w, m)) {
         ActPlanes a = act_planes(act, m, w->k);
-        if (w->glayout.type != TYPE_Q6_K && w->glayout.type != TYPE_Q5_K) a.q16 = nullptr;  // f16-MFMA GEMMs only
+        if (w->glayout.type == TYPE_Q8_0) a.q16 = nullptr;  // (the K-quant GEMMs read the f16 copy of the quants)
         e = act_q80(w->type) ? launch_quantize_q8_0(d_x, m, w->k, a, ctx->stream)
                                     : launch_quantize_q8k(d_x, m, w->k, a, ctx->stream);
         if (e != hipSuccess) return fail(AQ_ERR_HIP, "activation quantizer: %s", hipGetErrorString(e));
@@ -525,11 +525,14 @@ int aq_qmatmul_f32_device_noalloc(aq_ctx *ctx, const aq_qweight *w, const float 
     if ((rc = use_device(ctx->device))) return rc;
     const bool gemm = use_gemm(w, m);
     CallLayout L = call_layout(w, m, false, false, gemm);
-    if (L.total > FIXED_SCRATCH_BYTES)
+    // a K-quant GEMM splits K only as far as its partials fit
+    const size_t need = gemm && w->glayout.type != TYPE_Q8_0 ? L.ws : L.total;
+    if (need > FIXED_SCRATCH_BYTES)
         return fail(AQ_ERR_SHAPE, "m=%lld needs %zu bytes of scratch, more than the fixed %zu; use aq_qmatmul_f32_device",
-                    (long long)m, L.total, FIXED_SCRATCH_BYTES);
+                    (long long)m, need, FIXED_SCRATCH_BYTES);
+    const size_t room = std::min(L.total, FIXED_SCRATCH_BYTES) - L.ws;
     uint8_t *S = (uint8_t *)ctx->fixed_scratch;
-    return run_matmul(ctx, w, d_lhs, m, d_dst, S + L.act, nullptr, nullptr, S + L.ws, L.total - L.ws);
+    return run_matmul(ctx, w, d_lhs, m, d_dst, S + L.act, nullptr, nullptr, S + L.ws, room);
 }
 
 size_t aq_fixed_scratch_bytes(void) { return FIXED_SCRATCH_BYTES; }
@@ -594,10 +597,10 @@ int aq_qmatmul2_preq_device(aq_ctx *ctx, const aq_qweight *w1, const aq_qweight 
     if ((rc = use_device(ctx->device))) return rc;
     hipError_t e = hipErrorNotSupported;
     if (use_gemm(w1, m) && use_gemm(w2, m)) {
-        CallLayout L = call_layout(w2, m, false, false, true);  // the second GEMM's split-K partials
-        if ((rc = ensure_scratch(ctx, L.total))) return rc;
+        const size_t ws = gemm_pair_workspace_bytes(m, w2->n, k);  // the second GEMM's split-K partials
+        if ((rc = ensure_scratch(ctx, ws))) return rc;
         e = launch_gemm_pair(w1->glayout, w1->n, d_y1, w2->glayout, w2->n, d_y2, k, act_planes((void *)d_act, m, k), m,
-                             (uint8_t *)ctx->scratch + L.ws, L.total - L.ws, ctx->stream);
+                             ctx->scratch, ws, ctx->stream);
     }
     if (e == hipSuccess) return AQ_OK;
     if (e != hipErrorNotSupported) return fail(AQ_ERR_HIP, "paired gemm: %s", hipGetErrorString(e));

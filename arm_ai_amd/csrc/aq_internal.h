@@ -87,9 +87,9 @@ inline int groups_of(int type, int64_t k) {
 //   bsum16 [m][k/16]  the same bsums as f16 bits (exact: |bsum| <= 2048), the
 //                     A operand of the GEMM's f16 MFMA for the min term
 //   q16   [m][k]      the qs as f16 bits, the activation operand of the
-//                     f16-MFMA GEMMs (Q6_K, Q5_K); written by the Q8_K
-//                     quantizers when the pointer is set (paths that feed no
-//                     such GEMM clear it)
+//                     K-quant GEMMs, each four elements in the order 0, 2, 1,
+//                     3 (gemm_kq.h); written by the Q8_K quantizers when the
+//                     pointer is set (paths that feed no such GEMM clear it)
 struct ActPlanes {
     int8_t *qs;
     float *d;
@@ -195,14 +195,14 @@ hipError_t launch_mmv(const WLayout &w, int64_t n, int64_t k, const ActPlanes &a
                       int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s);
 // Prefill GEMM on MFMA (m > 8).  Returns hipErrorNotSupported for shapes it
 // does not take; the caller then uses launch_matvec.  ws: gemm_workspace_bytes
-// of scratch (split-K partials, summed by a second launch on the stream).
+// of scratch (split-K partials, summed by a second launch on the stream); with
+// less, the K-quant GEMMs split less.
 constexpr int GEMM_MAX_TILES = 1 << 20;
 hipError_t launch_gemm(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, int64_t m, float *y, int32_t *S,
                        int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s);
 // A Q4_K weight and a Q6_K / Q5_K weight of the same k on one activation
-// (with its f16 quants plane) in one launch, the first unsplit, the second
-// split over k as launch_gemm would (its partials in ws, gemm_workspace_bytes
-// of the second weight's shape, and its reduce launch after).
+// in one launch, the first unsplit, the second split over k (its partials in
+// ws, gemm_pair_workspace_bytes, and its reduce launch after).
 // hipErrorNotSupported when the types differ from that, the rows need more
 // than one launch, or the two together have more work items than the CUs
 // hold at once (the caller then runs launch_gemm twice).
@@ -211,13 +211,10 @@ hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLay
 // Workspace bytes launch_gemm needs for this shape, or (size_t)-1 if the
 // weight type / shape has no GEMM (the matvec then serves m > 8 too).
 size_t gemm_workspace_bytes(int type, int64_t m, int64_t n, int64_t k);
-// The Q6_K and Q5_K GEMM on f16 MFMA (k_gemm6.hip), reached through launch_gemm /
-// gemm_workspace_bytes.  It reads the activation quants as f16 from
-// ActPlanes::q16 when that is set (the quantizer wrote them), else converts
-// them into its workspace first; the workspace also holds the split-K partials.
-size_t gemm6_workspace_bytes(int64_t m, int64_t n, int64_t k);
-hipError_t launch_gemm6(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, int64_t m, float *y, int32_t *S,
-                        int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s);
+// Workspace that lets launch_gemm_pair split its second weight as far as it would.
+size_t gemm_pair_workspace_bytes(int64_t m, int64_t n2, int64_t k);
+// y[e] = part[0][e] + part[1][e] + ... of `total` elements, in split order.
+hipError_t launch_reduce(const float *part, float *y, int64_t total, int splits, hipStream_t s);
 // The Q8_0 GEMM on int8 MFMA (k_gemm8.hip), reached through launch_gemm /
 // gemm_workspace_bytes; its workspace holds the split-K partial tiles.
 size_t gemm8_workspace_bytes(int64_t m, int64_t n, int64_t k);
@@ -563,8 +560,9 @@ __device__ __forceinline__ void store_q8k_block64(const ActPlanes &a, int64_t ro
         uint32_t o[2];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)(int)(int8_t)((packed >> (16 * j)) & 0xffu));
-            const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)(int)(int8_t)((packed >> (16 * j + 8)) & 0xffu));
+            // elements 0, 2 then 1, 3 (the plane's pair order)
+            const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)(int)(int8_t)((packed >> (8 * j)) & 0xffu));
+            const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)(int)(int8_t)((packed >> (8 * j + 16)) & 0xffu));
             o[j] = lo | (hi << 16);
         }
         *(uint2 *)(a.q16 + e0) = make_uint2(o[0], o[1]);

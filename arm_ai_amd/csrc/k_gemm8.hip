@@ -298,7 +298,59 @@ int64_t gemm8_chunk_rows(int64_t m, int64_t k) {
     return m < cap ? m : cap;
 }
 
+// y = sum over splits (in split order) of the partial tiles; one thread per
+// output element of a tile row.  A kernel boundary, not a fence, makes the
+// partials visible: a device-scope fence per workgroup costs an L2
+// write-back on this GPU.
+// V consecutive columns of one tile row per thread (V = 4: 16-byte loads and
+// stores, where n % 4 == 0 and y is 16-byte aligned, so that the four stay in
+// one output row; the partial tiles are 128 columns wide).  Indices in 32
+// bits: the launcher checks that the tiles' elements fit.  The sum starts
+// from 0 and adds the parts in order, whatever V.
+template <int V>
+__global__ __launch_bounds__(256) void gemm_splitk_reduce(const float *__restrict__ part, float *__restrict__ y, int m,
+                                                          int n, int ntm, int gbm, int splits, int tiles) {
+    const int per_tile = gbm * G8T;
+    const int e = ((int)blockIdx.x * 256 + (int)threadIdx.x) * V;
+    if (e >= tiles * per_tile) return;
+    const int tile = e / per_tile;
+    const int w = e - tile * per_tile;
+    const int tn = tile / ntm, tm = tile - tn * ntm;
+    const int row = tm * gbm + w / G8T, c = tn * G8T + w % G8T;
+    if (row >= m || c >= n) return;
+    const float *src = part + (int64_t)tile * splits * per_tile + w;
+    float *dst = y + (int64_t)row * n + c;
+    if (V == 4 && c + 4 <= n) {
+        float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int s2 = 0; s2 < splits; s2++) {
+            const float4 t = *(const float4 *)(src + (int64_t)s2 * per_tile);
+            acc.x += t.x;
+            acc.y += t.y;
+            acc.z += t.z;
+            acc.w += t.w;
+        }
+        *(float4 *)dst = acc;
+    } else {
+        for (int j = 0; j < V && c + j < n; j++) {
+            float acc = 0.0f;
+            for (int s2 = 0; s2 < splits; s2++) acc += src[(int64_t)s2 * per_tile + j];
+            dst[j] = acc;
+        }
+    }
+}
+
 }  // namespace
+
+hipError_t launch_splitk_reduce(const float *part, float *y, int m, int n, int ntm, int gbm, int splits, int tiles,
+                                hipStream_t s) {
+    const int64_t elems = (int64_t)tiles * gbm * G8T;
+    if (elems + 4 * 256 > 0x7fffffff) return hipErrorInvalidValue;
+    if (n % 4 == 0 && (((uintptr_t)y | (uintptr_t)part) & 15) == 0)
+        gemm_splitk_reduce<4><<<(unsigned)((elems / 4 + 255) / 256), 256, 0, s>>>(part, y, m, n, ntm, gbm, splits, tiles);
+    else
+        gemm_splitk_reduce<1><<<(unsigned)((elems + 255) / 256), 256, 0, s>>>(part, y, m, n, ntm, gbm, splits, tiles);
+    return hipGetLastError();
+}
 
 size_t gemm8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || n <= 0 || k <= 0 || k % QK8_0 || k > (1 << 24)) return (size_t)-1;

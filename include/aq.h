@@ -21,11 +21,9 @@
  *    last message.
  *  - Weight type ids are GGUF/GGML dtype ids (Q4_0 = 2, Q5_0 = 6, Q8_0 = 8,
  *    Q2_K = 10, Q3_K = 11, Q4_K = 12, Q5_K = 13, Q6_K = 14).  Every type
- *    runs the batch-1..8 matvec.  For m > 8, Q4_K, Q5_K, Q6_K, Q8_0, Q4_0
- *    and Q5_0 run a prefill GEMM (Q4_0 and Q5_0 on an int8 copy that the
- *    upload expands into the Q8_0 layout, 34 bytes per 32 weights beside
- *    their 18- or 22-byte decode tiles);
- *    Q2_K and Q3_K run the matvec in passes of 8 rows.
+ *    runs the batch-1..8 matvec and, for m > 8, a prefill GEMM (Q4_0 and
+ *    Q5_0 on an int8 copy that the upload expands into the Q8_0 layout, 34
+ *    bytes per 32 weights beside their 18- or 22-byte decode tiles).
  *  - A weight is n rows (output features) by k columns (input features),
  *    row-major blocks, exactly candle's QTensor storage of shape (n, k).
  *  - Host-pointer entry points are synchronous at return.  Device-pointer
