@@ -5,8 +5,8 @@
 // :93 / :119 at prefill / decode).  Weights are uploaded once, repacked into
 // the HBM row-block tile layout (aq_internal.h), and every matmul runs on the context's
 // stream as either one matvec kernel that quantises the f32 activation itself
-// (m <= 8), or the activation quantizer kernel (Q8_K, or Q8_0 for Q8_0
-// weights) followed by the MFMA GEMM (m > 8).  Errors are status codes plus
+// (few rows), or the activation quantizer kernel (Q8_K, or Q8_0 for Q8_0
+// weights) followed by the MFMA GEMM.  Errors are status codes plus
 // a thread-local message;
 // nothing here aborts (the reference crate builds with panic = "abort",
 // Cargo.toml:33, which this library must not inherit).
@@ -207,7 +207,7 @@ CallLayout call_layout(const aq_qweight *w, int64_t m, bool host_io, bool dump, 
 }
 
 bool use_gemm(const aq_qweight *w, int64_t m) {
-    return m > 8 && gemm_workspace_bytes(w->glayout.type, m, w->n, w->k) != (size_t)-1;
+    return m >= gemm_min_rows(w->glayout.type) && gemm_workspace_bytes(w->glayout.type, m, w->n, w->k) != (size_t)-1;
 }
 // 2 or more rows of Q4_K / Q6_K without a GEMM: quantizer kernel, then the
 // matrix-core matvec
@@ -224,8 +224,8 @@ int check_mm(aq_ctx *ctx, const aq_qweight *w, int64_t m, int64_t k) {
     return AQ_OK;
 }
 
-// The matmul of d_x [m][k] into d_y on ctx->stream.  m > 8 with a GEMM for
-// the shape: the quantizer kernel writes the activation planes at `act`, then
+// The matmul of d_x [m][k] into d_y on ctx->stream.  Rows enough for a GEMM
+// (gemm_min_rows): the quantizer kernel writes the activation planes at `act`, then
 // the GEMM.  Other m >= 2 of Q4_K / Q6_K: the quantizer, then the
 // matrix-core matvec (passes of 8 rows).  Otherwise (m = 1, Q8_0): one matvec
 // launch that quantises d_x itself.
@@ -571,7 +571,7 @@ int aq_qmatmul_preq_device(aq_ctx *ctx, const aq_qweight *w, const void *d_act, 
     hipError_t e = hipErrorNotSupported;
     const bool gemm = use_gemm(w, m);
     CallLayout L = call_layout(w, m, false, false, gemm);
-    if ((gemm || use_mmv(w, m)) && (rc = ensure_scratch(ctx, L.total))) return rc;
+    if (L.total > L.ws && (gemm || use_mmv(w, m)) && (rc = ensure_scratch(ctx, L.total))) return rc;
     if (gemm) {
         e = launch_gemm(w->glayout, w->n, w->k, a, m, d_dst, nullptr, nullptr, (uint8_t *)ctx->scratch + L.ws,
                         L.total - L.ws, ctx->stream);

@@ -86,9 +86,9 @@ inline int groups_of(int type, int64_t k) {
 //   bsums [m][k/16]   i16 (Q8_K)
 //   bsum16 [m][k/16]  the same bsums as f16 bits (exact: |bsum| <= 2048), the
 //                     A operand of the GEMM's f16 MFMA for the min term
-//   q16   [m][k]      the qs as f16 bits, the activation operand of the
-//                     K-quant GEMMs, each four elements in the order 0, 2, 1,
-//                     3 (gemm_kq.h); written by the Q8_K quantizers when the
+//   q16   m * k       the qs as f16 bits, the activation operand of the
+//                     K-quant GEMMs, in the order in which their MFMAs read
+//                     it (q16_at); written by the Q8_K quantizers when the
 //                     pointer is set (paths that feed no such GEMM clear it)
 struct ActPlanes {
     int8_t *qs;
@@ -97,6 +97,7 @@ struct ActPlanes {
     int16_t *bsums;
     uint16_t *bsum16;
     uint16_t *q16 = nullptr;
+    int64_t m = 0;  // rows of the planes
 };
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -126,7 +127,24 @@ inline ActPlanes act_planes(void *base, int64_t m, int64_t k) {
     a.bsums = (int16_t *)(p + s.qs + s.d + s.d16);
     a.bsum16 = (uint16_t *)(p + s.qs + s.d + s.d16 + s.bsums);
     a.q16 = (uint16_t *)(p + s.qs + s.d + s.d16 + s.bsums + s.bsum16);
+    a.m = m;
     return a;
+}
+
+// Element offset in the q16 plane of the four elements 4 * l4 .. + 3 of block
+// b (stored in the order 0, 2, 1, 3) of a row.  Rows go in tiles of 32 (the
+// last one of fewer, `rows`), and within a tile the 16 elements 32 S + 16 h ..
+// of a block, for the halves h and the tile's rows, lie side by side: the two
+// fragments (8 elements a lane: half h, row r) that v_mfma_f32_32x32x16_f16
+// takes of sub-block S.  A wavefront's fragment is then 32 whole sectors in
+// lane order, and what a quantizer writes of one row comes in sectors too
+// (with fragments alone side by side it was 16 bytes apart from the next row's:
+// 512 x 14336 x 4096 74.2 us against 72.0 row-major).
+__host__ __device__ inline int64_t q16_at(int64_t row, int64_t m, int64_t k, int64_t b, int l4) {
+    const int64_t t0 = row & ~(int64_t)31;
+    const int64_t rows = m - t0 < 32 ? m - t0 : 32;
+    const int S = l4 >> 3, h = (l4 >> 2) & 1;
+    return t0 * k + (((b * 8 + S) * 2 + h) * rows + (row - t0)) * 16 + 4 * (l4 & 3);
 }
 
 // ---------------------------------------------------------------------------
@@ -211,6 +229,8 @@ hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLay
 // Workspace bytes launch_gemm needs for this shape, or (size_t)-1 if the
 // weight type / shape has no GEMM (the matvec then serves m > 8 too).
 size_t gemm_workspace_bytes(int type, int64_t m, int64_t n, int64_t k);
+// The fewest rows for which launch_gemm is the faster path.
+int gemm_min_rows(int type);
 // Workspace that lets launch_gemm_pair split its second weight as far as it would.
 size_t gemm_pair_workspace_bytes(int64_t m, int64_t n2, int64_t k);
 // y[e] = part[0][e] + part[1][e] + ... of `total` elements, in split order.
@@ -560,12 +580,11 @@ __device__ __forceinline__ void store_q8k_block64(const ActPlanes &a, int64_t ro
         uint32_t o[2];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            // elements 0, 2 then 1, 3 (the plane's pair order)
             const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)(int)(int8_t)((packed >> (8 * j)) & 0xffu));
             const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)(int)(int8_t)((packed >> (8 * j + 16)) & 0xffu));
             o[j] = lo | (hi << 16);
         }
-        *(uint2 *)(a.q16 + e0) = make_uint2(o[0], o[1]);
+        *(uint2 *)(a.q16 + q16_at(row, a.m, k, sb, lane)) = make_uint2(o[0], o[1]);
     }
     if ((lane & 3) == 0) {
         a.bsums[row * (k / 16) + sb * 16 + (lane >> 2)] = (int16_t)bsum;

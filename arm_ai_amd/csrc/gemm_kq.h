@@ -42,7 +42,9 @@
 // so a lane reads whole 16-byte pieces of its own column.
 //   * The activation rows (f16 quants, bsums, d) go global -> LDS by
 //     buffer-to-LDS copies into two stages, one per half of a super-block,
-//     issued one half ahead; 16-byte chunks are XOR-swizzled by the row.
+//     issued one half ahead; the plane is in fragment order, so a copy is one
+//     fragment and a fragment read one conflict-free ds_read at a constant
+//     offset.
 //   * The weights go straight into registers, one super-block ahead.
 //   * One s_waitcnt vmcnt and one barrier start each half.  Loads past the
 //     last super-block go through an empty descriptor.
@@ -61,7 +63,7 @@ struct KqParams {
     const uint16_t *wd;  // Q6_K, Q2_K: d plane
     int64_t rb_stride;
     int ng;              // super-blocks per row
-    const uint16_t *x16;  // activation quants as f16 [m][k] (pair order)
+    const uint16_t *x16;  // activation quants as f16 (q16_at)
     const float *xd;      // [m][ng]
     const uint16_t *xbs;  // bsums as f16 [m][k/16]
     float *y;             // [m][n], or with splits > 1 the partials [splits][m][n]
@@ -74,7 +76,9 @@ struct KqParams {
 struct KqForm {
     int rows, cols;
 };
-constexpr KqForm KQ_FORMS[] = {{32, 128}, {64, 128}, {128, 256}, {128, 128}};
+// 4, 5: few rows, 4 or 8 wavefronts over K (d of their rows in LDS, 128 bytes a super-block)
+constexpr KqForm KQ_FORMS[] = {{32, 128}, {64, 128}, {128, 256}, {128, 128}, {32, 32}, {32, 32}};
+constexpr int KQ_FEW_MAX_NG = 256;  // super-blocks of a split
 hipError_t launch_kq_q4k(const KqParams &p, int form, bool dump, hipStream_t s);
 hipError_t launch_kq_q5k(const KqParams &p, int form, bool dump, hipStream_t s);
 hipError_t launch_kq_q6k(const KqParams &p, int form, bool dump, hipStream_t s);
@@ -343,6 +347,22 @@ __device__ __forceinline__ void operands(const W<TYPE> &v, const Consts<TYPE> &c
     if constexpr (TYPE == TYPE_Q6_K) b[1] = __builtin_bit_cast(v8h, r2);
 }
 
+// The min product's operand: B[g][n] = the min of bsum group g = 8 h + e
+// (Q4_K, Q5_K: of its sub-block).
+template <int TYPE>
+__device__ __forceinline__ v8h min_operand(const Scales &z) {
+    u32x4 bm;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        if constexpr (TYPE == TYPE_Q2_K)
+            bm[e] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, z.mn[e >> 1], (e & 1) ? 0x04030402u : 0x04010400u)) -
+                           splat(1024.0f));
+        else
+            bm[e] = as_u32(pair_of_byte(z.mn[0], e));
+    }
+    return __builtin_bit_cast(v8h, bm);
+}
+
 // MFMA step J of a super-block: half I of sub-block S.  The sub-blocks that
 // share dwords follow each other, so that w >> 8 is formed once.
 template <int TYPE, int J>
@@ -359,7 +379,7 @@ struct Step {
 template <int MT>
 struct Lds {
     static constexpr int ROWS = 32 * MT;
-    static constexpr int QS = ROWS * 256;  // f16 quants [rows][128], chunk c of row r at c ^ (r & 15)
+    static constexpr int QS = ROWS * 256;  // f16 quants: fragments [row tile][8][lane]
     static constexpr int BS = 2 * QS;      // bsums [rows][16] f16
     static constexpr int DX = BS + ROWS * 32;  // d [rows] f32 (a copy writes 256 bytes)
     static constexpr int BYTES = DX + (ROWS * 4 < 256 ? 256 : ROWS * 4);
@@ -386,19 +406,19 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
     const int h = lane >> 5, l32 = lane & 31;
     const int ng = p.ng, k = p.k;
 
-    // activation copies: instruction i of wave w fills the LDS bytes of rows
-    // r = 4 (CI w + i) + lane / 16, chunk position lane % 16 holding the
-    // half's chunk (lane % 16) ^ (r & 15).  Rows past m lie past the range and
-    // read zeros (the scalar offset, which the range check leaves out, stays
-    // inside a row).
+    // activation copies: a wave copies CI fragments of one row tile per half.
+    // Rows past m read zeros (the scalar offset, which the range check leaves
+    // out, stays inside the tile).
     const rsrc_t rq = buf_rsrc(p.x16, (uint32_t)((int64_t)p.m * k * 2));
     const rsrc_t rdx = buf_rsrc(p.xd, (uint32_t)((int64_t)p.m * ng * 4));
     const rsrc_t rbs = buf_rsrc(p.xbs, (uint32_t)((int64_t)p.m * (k / 16) * 2));
     const rsrc_t rnone = buf_rsrc(p.x16, 0u);
     constexpr int CI = 8 * MT / NW;  // copies per wave and stage
-    const int r0 = 4 * CI * wave + (lane >> 4);
-    const uint32_t qrow = (uint32_t)((m0 + r0) * k * 2);
-    uint32_t qchunk = (uint32_t)(16 * ((lane & 15) ^ (r0 & 15)));  // of copy i: ^ 64 (i & 3)
+    static_assert(8 % CI == 0);
+    const int trow = m0 + 32 * (CI * wave / 8);  // the tile's first row
+    const int trows = min(32, p.m - trow);       // (none: every lane past the range)
+    const uint32_t qoff = l32 < trows ? (uint32_t)(trow * k * 2 + (h * trows + l32) * 32) : BUF_OOB;
+    const int sbytes = 64 * max(trows, 0);       // of a sub-block
     // bsums: 32 rows per instruction (two lanes a row), wave w those of rows
     // 32 w ..; d: 64 rows per instruction, from wave 3 down.  Every wave
     // issues two small copies, so that all wait on the same counts; the spare
@@ -442,11 +462,10 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
         const int b = kb0 + i;
         const bool live = i < nit;
         const rsrc_t r1 = live ? rq : rnone;
-        opaque(qchunk);
 #pragma unroll
         for (int c = 0; c < CI; c++)
-            buf_to_lds16(r1, lds + HF * L::QS + 1024 * (CI * wave + c),
-                         (qchunk ^ (uint32_t)(64 * (c & 3))) + (qrow + (uint32_t)(8 * c * k)), b * 512 + 256 * HF);
+            buf_to_lds16(r1, lds + HF * L::QS + 1024 * (CI * wave + c), qoff,
+                         (b * 8 + 4 * HF + (CI * wave + c) % 8 / 2) * sbytes + 16 * (c & 1));
         if constexpr (HF == 1) {
             if constexpr (MIN) {
                 const int bw = wave < MT ? wave : 0;  // (spare waves copy rows 0..31 of the tile again)
@@ -466,7 +485,7 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
 #pragma unroll
             for (int r = 0; r < 16; r++) yacc[t][u][r] = 0.0f;
 
-    uint32_t aoff = (uint32_t)(l32 * 256 + 16 * ((2 * h) ^ (l32 & 15)));  // this lane's fragment of step 0, row tile 0
+    const uint8_t *frag = lds + 16 * lane;  // this lane's part of fragment 0, row tile 0
     WT v[NT];
     auto super_block = [&](int i) {
         // This wave's copies of the half have landed (those of the other half
@@ -479,7 +498,6 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
             wait_vmcnt<HF == 0 ? PIECES1 : HEADS + PIECES0>();
             stage_barrier();
             issue(HF == 0 ? i : i + 1, std::integral_constant<int, 1 - HF>{});
-            opaque(aoff);
         };
         enter(std::integral_constant<int, 0>{});
         v16f acc[MT][NT];
@@ -511,10 +529,9 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
         auto build = [&](auto JC) {
             constexpr int J = decltype(JC)::value;
             using P = Step<TYPE, J>;
-            // the half's chunk 4 (S & 3) + 2 h + I of row 32 t + l32
-            const uint8_t *row = lds + (J >> 3) * L::QS + (aoff ^ (uint32_t)(16 * (4 * (P::S & 3) + P::I)));
 #pragma unroll
-            for (int t = 0; t < MT; t++) a[J & 1][t] = *(const v8h *)(row + 32 * 256 * t);
+            for (int t = 0; t < MT; t++)
+                a[J & 1][t] = *(const v8h *)(frag + (J >> 3) * L::QS + 8192 * t + 1024 * ((2 * P::S + P::I) & 7));
 #pragma unroll
             for (int u = 0; u < NT; u++) {
                 if constexpr (P::I == 0) c[u][J % P::SHARE] = consts<TYPE>(z[u], P::S);
@@ -583,21 +600,7 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
         v8h bmn[NT];
         if constexpr (MIN) {
 #pragma unroll
-            for (int u = 0; u < NT; u++) {
-                // B[g][n] = the min of group g = 8 h + e (Q4_K, Q5_K: of its sub-block)
-                u32x4 bm;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    if constexpr (TYPE == TYPE_Q2_K) {
-                        const uint32_t w = z[u].mn[e >> 1];
-                        bm[e] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, w, (e & 1) ? 0x04030402u : 0x04010400u)) -
-                                       splat(1024.0f));
-                    } else {
-                        bm[e] = as_u32(pair_of_byte(z[u].mn[0], e));
-                    }
-                }
-                bmn[u] = __builtin_bit_cast(v8h, bm);
-            }
+            for (int u = 0; u < NT; u++) bmn[u] = min_operand<TYPE>(z[u]);
         }
         constexpr int NSM = MT * NT > 1 ? 2 : 1;
         v16f sm[NSM];
@@ -660,6 +663,148 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// Few rows (a tile of 32).  The time is the weight stream's, and a column's
+// operands feed one MFMA each, so what fills the chip is many wavefronts with
+// a short chain each: the NW wavefronts of a workgroup share 32 columns and
+// take every NW-th super-block, with no LDS stage and no barrier in between
+// (the activation fragments come from the L2 in whole lines, one super-block
+// ahead like the weights), then add their sums through LDS in wavefront order.
+// ---------------------------------------------------------------------------
+template <int TYPE, int NW>
+__device__ __forceinline__ void few_body(const KqParams &p, float *dx, float *red, int bid) {
+    constexpr bool MIN = TYPE == TYPE_Q4_K || TYPE == TYPE_Q5_K || TYPE == TYPE_Q2_K;
+    constexpr int ND = TYPE == TYPE_Q6_K ? 2 : 1;
+    const int xcd = bid % NXCD, local = bid / NXCD;
+    const int item = xcd * p.per_xcd + local;
+    if (local >= p.per_xcd || item >= p.items) return;  // uniform over the workgroup
+    const int tile = item / p.splits, split = item - tile * p.splits;
+    const int tn = tile / p.ntm, m0 = 32 * (tile - tn * p.ntm);
+    const int rows = min(32, p.m - m0);
+    const int ng = p.ng, k = p.k;
+    const int kb0 = split * p.kbs, kb1 = min(ng, kb0 + p.kbs);
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, l32 = lane & 31;
+
+    const rsrc_t rq = buf_rsrc(p.x16, (uint32_t)((int64_t)p.m * k * 2));
+    const rsrc_t rbs = buf_rsrc(p.xbs, (uint32_t)((int64_t)p.m * (k / 16) * 2));
+    const rsrc_t rnone = buf_rsrc(p.x16, 0u);
+    const uint32_t qoff = l32 < rows ? (uint32_t)(m0 * k * 2 + (h * rows + l32) * 32) : BUF_OOB;
+    const uint32_t bsoff = l32 < rows ? (uint32_t)(((m0 + l32) * (k / 16) + 8 * h) * 2) : BUF_OOB;
+    const int sbytes = 64 * rows;  // of a sub-block
+    const int nrb = (p.n + RB - 1) / RB, rb0 = 4 * tn, rb_here = min(4, nrb - rb0);
+    const rsrc_t rw = buf_rsrc(p.w + (int64_t)rb0 * p.rb_stride, (uint32_t)(rb_here * p.rb_stride));
+    constexpr int DB = TYPE == TYPE_Q2_K ? 4 : 2;  // bytes per d-plane entry
+    const rsrc_t rwd = (TYPE == TYPE_Q6_K || TYPE == TYPE_Q2_K)
+                           ? buf_rsrc((const uint8_t *)p.wd + (int64_t)rb0 * ng * RB * DB, (uint32_t)(rb_here * ng * RB * DB))
+                           : rw;
+    const uint32_t woff[1] = {(uint32_t)((l32 >> 3) * p.rb_stride + (l32 & 7) * 16)};
+    const uint32_t doff[1] = {(uint32_t)((l32 >> 3) * ng * RB + (l32 & 7))};
+
+    // first super-block's loads, then d of the tile's rows into LDS [super-block][row]
+    W<TYPE> v[1];
+    u32x4 a[16], bs = {0, 0, 0, 0};
+    int b = kb0 + wave;
+    {
+        const bool live = b < kb1;
+        const rsrc_t r4 = live ? rw : rnone, r5 = live ? rwd : rnone, r1 = live ? rq : rnone;
+        load_all<TYPE, 1>(v, r4, r5, woff, doff, h, b);
+#pragma unroll
+        for (int f = 0; f < 16; f++) a[f] = ld16(r1, qoff, (b * 8 + f / 2) * sbytes + 16 * (f & 1));
+        if constexpr (MIN) bs = ld16(live ? rbs : rnone, bsoff, b * 32);
+    }
+    for (int e = tid; e < 32 * (kb1 - kb0); e += 64 * NW) {
+        const int r = e & 31, g = kb0 + (e >> 5);
+        dx[e] = r < rows ? p.xd[(int64_t)(m0 + r) * ng + g] : 0.0f;
+    }
+    lds_barrier();
+
+    v16f y;
+#pragma unroll
+    for (int r = 0; r < 16; r++) y[r] = 0.0f;
+    uint32_t magic = 0x64006400u;
+    opaque(magic);
+    for (; b < kb1; b += NW) {  // uniform over the wavefront
+        const int nb = b + NW;
+        const bool more = nb < kb1;
+        const rsrc_t r4 = more ? rw : rnone, r5 = more ? rwd : rnone, r1 = more ? rq : rnone;
+        const Scales z = unpack_scales<TYPE>(v[0], h);
+        const uint32_t dd = d_word<TYPE>(v[0]);
+        load_head<TYPE>(v[0], r4, r5, woff[0], doff[0], nb);
+        v16f acc;
+        Consts<TYPE> c[Step<TYPE, 0>::SHARE];
+        auto step = [&](auto JC) {
+            constexpr int J = decltype(JC)::value;
+            using P = Step<TYPE, J>;
+            constexpr int F = 2 * P::S + P::I;
+            if constexpr (P::I == 0) c[J % P::SHARE] = consts<TYPE>(z, P::S);
+            v8h w[ND];
+            operands<TYPE, P::S>(v[0], c[J % P::SHARE], P::I, magic, w);
+#pragma unroll
+            for (int g = 0; g < ND; g++) {
+                const v16f zero = {0};
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[F]), w[g], J == 0 && g == 0 ? zero : acc, 0, 0, 0);
+            }
+            a[F] = ld16(r1, qoff, (nb * 8 + P::S) * sbytes + 16 * P::I);
+            if constexpr (P::LAST) load_after<TYPE, P::S>(v[0], r4, woff[0], h, nb);
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 4>{});
+        step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{});
+        step(std::integral_constant<int, 7>{});
+        step(std::integral_constant<int, 8>{});
+        step(std::integral_constant<int, 9>{});
+        step(std::integral_constant<int, 10>{});
+        step(std::integral_constant<int, 11>{});
+        step(std::integral_constant<int, 12>{});
+        step(std::integral_constant<int, 13>{});
+        step(std::integral_constant<int, 14>{});
+        step(std::integral_constant<int, 15>{});
+        v16f sm;
+        if constexpr (MIN) {
+            const v16f zero = {0};
+            sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bs), min_operand<TYPE>(z), zero, 0, 0, 0);
+            bs = ld16(more ? rbs : rnone, bsoff, nb * 32);
+        }
+        const float dw = f16_bits_to_f32(dd) * (TYPE == TYPE_Q6_K ? 16.0f : 1.0f), dmw = f16_bits_to_f32(dd >> 16);
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++) {
+            const v4f dx4 = *(const v4f *)(dx + 32 * (b - kb0) + 8 * g4 + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = 4 * g4 + e;
+                if constexpr (MIN) y[r] = __builtin_fmaf(dx4[e], __builtin_fmaf(-dmw, sm[r], dw * acc[r]), y[r]);
+                else y[r] = __builtin_fmaf(dw * dx4[e], acc[r], y[r]);
+            }
+        }
+    }
+
+    // red [wavefront][row of 32][column of 32]
+#pragma unroll
+    for (int r = 0; r < 16; r++) red[(wave * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * 32 + l32] = y[r];
+    lds_barrier();
+    float *out = p.y + (p.splits > 1 ? (int64_t)split * p.m * p.n : 0);
+    for (int e = tid; e < 32 * rows; e += 64 * NW) {
+        const int r = e >> 5, col = 32 * tn + (e & 31);
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) sum += red[w * 1024 + e];
+        if (col < p.n) out[(int64_t)(m0 + r) * p.n + col] = sum;
+    }
+}
+
+template <int TYPE, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void few_kernel(KqParams p) {
+    extern __shared__ __align__(16) uint8_t dyn[];  // [NW][32][32] f32, then d
+    few_body<TYPE, NW>(p, (float *)(dyn + NW * 4096), (float *)dyn, (int)blockIdx.x);
+}
+
 template <int TYPE, int MT, int NT, int NW, int OCC, bool DUMP>
 __global__ __launch_bounds__(64 * NW, OCC) void kernel(KqParams p) {
     __shared__ __align__(16) uint8_t lds[Lds<MT>::BYTES];
@@ -685,6 +830,8 @@ hipError_t launch(const KqParams &p, int form, bool dump, hipStream_t s) {
     else if (form == 1) kernel<TYPE, 2, 1, 4, TYPE == TYPE_Q6_K ? 2 : 3, false><<<grid, 256, 0, s>>>(p);
     else if (form == 2) kernel<TYPE, 4, 1, 8, 2, false><<<grid, 512, 0, s>>>(p);
     else if (form == 3) kernel<TYPE, 4, 1, 4, 2, false><<<grid, 256, 0, s>>>(p);
+    else if (form == 4) few_kernel<TYPE, 4><<<grid, 256, 4 * 4096 + 128 * p.kbs, s>>>(p);
+    else if (form == 5) few_kernel<TYPE, 8><<<grid, 512, 8 * 4096 + 128 * p.kbs, s>>>(p);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }

@@ -49,34 +49,44 @@ struct Plan {
 };
 
 // The tile form and K split of least estimated time.  Per form, measured on
-// Q4_K over 1024..14336 columns, K of 2048..14336 and 9..1024 rows: the time
-// of one super-block of a workgroup alone on its CU (bound by its own chain),
-// its share when the CU is full (bound by VALU and MFMA issue), and the
-// workgroups a CU holds.  A split adds the reduce launch and one write and
-// read of its partials.  The order of the measured times is the estimate's:
-// 512 x 14336 x 4096 78 us as 128 x 256, 90 as 64 x 128; 512 x 5632 x 2048 28
-// as 64 x 128, 33 (two splits) as 128 x 256; 64 x 4096 x 4096 16.0 as 32 x
-// 128 in four splits, 19.2 in two, 16.8 as 64 x 128.
+// Q4_K over 512..14336 columns, K of 1024..14336 and 9..1024 rows: the time of
+// one step of a workgroup alone on its CU (bound by its own chain), its share
+// when the CU holds more (bound by VALU and MFMA issue), the workgroups a CU
+// holds, and the super-blocks of a step (the few-row forms' wavefronts take
+// one each).  A split adds the reduce launch and one write and read of its
+// partials.  Rows x columns x K, with the quantizer launch:
+//   512 x 14336 x 4096  128 x 256 tiles 78 us, 64 x 128 90
+//   512 x 5632 x 2048   64 x 128 28 us, 128 x 256 in two splits 33
+//   128 x 4096 x 4096   few rows 17.5 us, 64 x 128 in four splits 21.1
+//   16 x 14336 x 4096   few rows, four wavefronts 14.6 us, eight 17.7, 32 x 128 in four splits 16.3
+//   16 x 4096 x 14336   few rows, eight wavefronts in two splits 17.1 us, unsplit 19.0
 struct FormCost {
     float alone, full;
-    int slots;
+    int slots, blocks;
 };
-constexpr FormCost COST[] = {{1.0f, 0.82f, 2}, {1.3f, 1.25f, 3}, {4.3f, 4.3f, 1}, {2.85f, 2.28f, 2}};
+constexpr FormCost COST[] = {{1.3f, 0.82f, 2, 1},  {1.5f, 1.25f, 3, 1}, {4.3f, 4.3f, 1, 1},
+                             {2.85f, 2.28f, 2, 1}, {1.08f, 1.12f, 3, 4}, {1.93f, 3.0f, 1, 8}};
+constexpr int NFORMS = 6;
 
 Plan kq_plan(int type, int64_t m, int64_t n, int64_t k) {
     const int ng = (int)(k / QK_K);
     const float weight = type == TYPE_Q6_K ? 1.4f : type == TYPE_Q5_K ? 1.1f : 1.0f;  // time of a step against Q4_K's
+    // up to 8 rows no split: those calls never needed a workspace
+    const int most_splits = m <= 8 ? 1 : 16;
     Plan best{};
     float best_us = 0.0f;
-    for (int form = 0; form < 4; form++) {
+    for (int form = 0; form < NFORMS; form++) {
         const KqForm f = KQ_FORMS[form];
+        const FormCost &t = COST[form];
         const int64_t ntm = (m + f.rows - 1) / f.rows, ntn = (n + f.cols - 1) / f.cols;
         if (form == 2 && (int64_t)(f.cols / RB) * slabs_of(type) * ng * 128 >= ((int64_t)1 << 31)) continue;  // 32-bit offsets in a tile
-        for (int splits = 1; splits <= 16 && splits * 2 <= std::max(ng, 2); splits *= 2) {
+        for (int splits = 1; splits <= most_splits && splits * 2 <= std::max(ng, 2); splits *= 2) {
             const int kbs = (ng + splits - 1) / splits, ns = (ng + kbs - 1) / kbs;
+            if (t.blocks > 1 && kbs > KQ_FEW_MAX_NG) continue;
             const float c = (float)((ntm * ntn * ns + 255) / 256);  // workgroups of the busiest CU
-            const float rounds = std::max(COST[form].alone * std::ceil(c / COST[form].slots), COST[form].full * c);
-            const float us = weight * kbs * rounds + (ns > 1 ? 1.5f + 8.0f * ns * (float)m * (float)n / 3.5e6f : 0.0f);
+            const float step = c <= 1.0f ? t.alone : std::max(t.alone * std::ceil(c / t.slots), t.full * c);
+            const float us = weight * ((kbs + t.blocks - 1) / t.blocks) * step +
+                             (ns > 1 ? 2.5f + 8.0f * ns * (float)m * (float)n / 3.5e6f : 0.0f);
             if (best_us == 0.0f || us < best_us) {
                 best_us = us;
                 best = {form, (int)ntm, (int)ntn, ns, kbs, ns > 1 ? (size_t)ns * m * n * 4 : 0};
@@ -95,6 +105,11 @@ Plan kq_plan_in(int type, int64_t m, int64_t n, int64_t k, size_t room) {
         g.kbs = (ng + g.splits - 1) / g.splits;
         g.splits = (ng + g.kbs - 1) / g.kbs;
         g.ws = g.splits > 1 ? (size_t)g.splits * m * n * 4 : 0;
+        if (COST[g.form].blocks > 1 && g.kbs > KQ_FEW_MAX_NG) {
+            g.form = 0;
+            g.ntm = (int)((m + 31) / 32);
+            g.ntn = (int)((n + 127) / 128);
+        }
     }
     return g;
 }
@@ -135,6 +150,14 @@ KqParams kq_params(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, i
 }
 
 }  // namespace
+
+// Q5_K, Q2_K and Q3_K have no matrix-core matvec, and the dot4 matvec's time
+// grows with the rows: from three rows the GEMM's few-row forms are faster
+// (Q3_K 14336 x 4096: 2 rows 12.9 us against 15.3, 4 rows 20.4 against 15.3, 8
+// rows 35 against 15.4; 5632 x 2048: 7.4 against 8.8, 11.2 against 8.7, 18.8
+// against 8.7).  The matrix-core matvec keeps Q4_K and Q6_K up to its 8 rows
+// (11.0 against 14.1 at 8 x 14336 x 4096, 8.3 against 8.9 at 8 x 5632 x 2048).
+int gemm_min_rows(int type) { return type == TYPE_Q5_K || type == TYPE_Q2_K || type == TYPE_Q3_K ? 3 : 9; }
 
 hipError_t launch_reduce(const float *part, float *y, int64_t total, int splits, hipStream_t s) {
     if (total % 4 == 0 && (((uintptr_t)y | (uintptr_t)part) & 15) == 0)

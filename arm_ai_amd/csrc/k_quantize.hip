@@ -14,13 +14,14 @@ namespace aq {
 // (q8k_block_wave, the fused prologues' code): four blocks per 256-thread
 // workgroup.
 template <bool VEC>
-__global__ __launch_bounds__(256) void quantize_q8k_kernel(const float *__restrict__ x, int64_t nblocks,
+__global__ __launch_bounds__(256) void quantize_q8k_kernel(const float *__restrict__ x, int64_t nblocks, int64_t k,
                                                            ActPlanes a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t bi = (int64_t)blockIdx.x * 4 + wave;
     if (bi >= nblocks) return;  // uniform over the wavefront
-    // (blocks, bsums and d lie one after the other over the rows: no row index)
+    // (blocks, bsums and d lie one after the other over the rows; only the f16
+    // plane needs the row)
     const int64_t e0 = bi * QK_K + 4 * lane;
     float v[4];
     if (VEC) {
@@ -36,7 +37,9 @@ __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float *__restri
     int bsum;
     float d;
     const uint32_t packed = q8k_block_wave(v, lane, &bsum, &d);
-    store_q8k_block64(a, 0, 0, bi, lane, packed, bsum, d);
+    const uint32_t nb = (uint32_t)(k / QK_K);
+    const int64_t row = !a.q16 ? 0 : nblocks <= 0x7fffffff ? (uint32_t)bi / nb : bi / nb;
+    store_q8k_block64(a, row, k, bi - row * nb, lane, packed, bsum, d);
 }
 
 // Eight lanes per 32-element block, 32 blocks per workgroup.
@@ -74,9 +77,9 @@ hipError_t launch_quantize_q8k(const float *x, int64_t m, int64_t k, ActPlanes a
     const int64_t grid = (nblocks + 3) / 4;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     if (((uintptr_t)x & 15) == 0)
-        quantize_q8k_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
+        quantize_q8k_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
     else
-        quantize_q8k_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
+        quantize_q8k_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
     return hipGetLastError();
 }
 

@@ -21,9 +21,10 @@
  *    last message.
  *  - Weight type ids are GGUF/GGML dtype ids (Q4_0 = 2, Q5_0 = 6, Q8_0 = 8,
  *    Q2_K = 10, Q3_K = 11, Q4_K = 12, Q5_K = 13, Q6_K = 14).  Every type
- *    runs the batch-1..8 matvec and, for m > 8, a prefill GEMM (Q4_0 and
- *    Q5_0 on an int8 copy that the upload expands into the Q8_0 layout, 34
- *    bytes per 32 weights beside their 18- or 22-byte decode tiles).
+ *    runs a matvec at m = 1 and small batches, and a prefill GEMM for more
+ *    rows (m > 8; Q5_K, Q2_K and Q3_K m > 2; Q4_0 and Q5_0 on an int8 copy
+ *    that the upload expands into the Q8_0 layout, 34 bytes per 32 weights
+ *    beside their 18- or 22-byte decode tiles).
  *  - A weight is n rows (output features) by k columns (input features),
  *    row-major blocks, exactly candle's QTensor storage of shape (n, k).
  *  - Host-pointer entry points are synchronous at return.  Device-pointer
@@ -157,8 +158,8 @@ int aq_quantize_q8_0(aq_ctx *ctx, const float *x, int64_t m, int64_t k, void *ou
  *   Q6_K: S = sum_j sc_j * sum_{e in sub-block j} q6_e*qx_e, Smin = 0
  *   Q8_0: S = sum_{32} qw*qx per 32-block,                    Smin = 0
  *   Q4_0: S = sum_{32} (q-8)*qx per 32-block,                 Smin = 0
- * computed by the same kernel code as aq_qmatmul_f32 (batch <= 8 path)
- * or the prefill GEMM (m > 8) with an integer epilogue.  Host buffers. */
+ * computed by the same kernel code as aq_qmatmul_f32 (the matvec or the
+ * prefill GEMM, by the number of rows) with an integer epilogue.  Host buffers. */
 int aq_qmatmul_block_sums(aq_ctx *ctx, const aq_qweight *w, const float *lhs, int64_t m,
                           int64_t k, int32_t *S, int32_t *Smin);
 

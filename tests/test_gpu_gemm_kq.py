@@ -24,6 +24,15 @@ def test_tile_edges(ctx, t, n, k, m):
     check_matmul(ctx, S.make_weight(t, n, k, rng=rng), S.make_activation(m, k, seed=m))
 
 
+# the few-row forms: four and eight wavefronts over K, with and without a
+# split, K from one super-block (idle wavefronts) to an odd count
+@pytest.mark.parametrize("t", KQ)
+@pytest.mark.parametrize("n,k,m", [(33, 256, 3), (70, 768, 5), (1000, 2304, 8), (2048, 5632, 17), (520, 3840, 40)])
+def test_few_rows(ctx, t, n, k, m):
+    rng = np.random.default_rng(n + 3 * m)
+    check_matmul(ctx, S.make_weight(t, n, k, rng=rng), S.make_activation(m, k, seed=m + 1))
+
+
 # many row and column tiles: the 128 x 256 form (outputs only: the dump has its own form)
 @pytest.mark.parametrize("t", KQ)
 def test_large_tiles(ctx, t):
