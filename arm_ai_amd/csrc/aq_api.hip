@@ -207,7 +207,7 @@ CallLayout call_layout(const aq_qweight *w, int64_t m, bool host_io, bool dump, 
 }
 
 bool use_gemm(const aq_qweight *w, int64_t m) {
-    return m >= gemm_min_rows(w->glayout.type) && gemm_workspace_bytes(w->glayout.type, m, w->n, w->k) != (size_t)-1;
+    return m >= gemm_min_rows(w->glayout.type, w->k) && gemm_workspace_bytes(w->glayout.type, m, w->n, w->k) != (size_t)-1;
 }
 // 2 or more rows of Q4_K / Q6_K without a GEMM: quantizer kernel, then the
 // matrix-core matvec
@@ -234,7 +234,6 @@ int run_matmul(aq_ctx *ctx, const aq_qweight *w, const float *d_x, int64_t m, fl
     hipError_t e;
     if (use_gemm(w, m)) {
         ActPlanes a = act_planes(act, m, w->k);
-        if (w->glayout.type == TYPE_Q8_0) a.q16 = nullptr;  // (the K-quant GEMMs read the f16 copy of the quants)
         e = act_q80(w->type) ? launch_quantize_q8_0(d_x, m, w->k, a, ctx->stream)
                                     : launch_quantize_q8k(d_x, m, w->k, a, ctx->stream);
         if (e != hipSuccess) return fail(AQ_ERR_HIP, "activation quantizer: %s", hipGetErrorString(e));

@@ -147,6 +147,20 @@ __host__ __device__ inline int64_t q16_at(int64_t row, int64_t m, int64_t k, int
     return t0 * k + (((b * 8 + S) * 2 + h) * rows + (row - t0)) * 16 + 4 * (l4 & 3);
 }
 
+// Q8_0 activations: the q16 plane's bytes hold what the Q8_0 GEMM reads, the
+// quants as tiles of 32 rows (fewer in the last) of [block][row][32 bytes],
+// and after them (dt_plane) d in f32 as tiles of [block][32 rows].  Both fit
+// from four rows on (the fewest the GEMM takes): 36 bytes per block and row,
+// tiles rounded up, against 64.
+constexpr int Q8_MIN_ROWS = 4;
+constexpr int Q8_FEW_MAX_GROUPS = 112;  // groups of a split in the GEMM's few-row forms (d in LDS, 1 KiB a group)
+__host__ __device__ inline int64_t q8_at(int64_t row, int64_t m, int64_t k, int64_t b) {  // bytes
+    const int64_t t0 = row & ~(int64_t)31;
+    return t0 * k + (b * (m - t0 < 32 ? m - t0 : 32) + (row - t0)) * 32;
+}
+__host__ __device__ inline float *dt_plane(const ActPlanes &a, int64_t k) { return (float *)((uint8_t *)a.q16 + a.m * k); }
+__host__ __device__ inline int64_t dt_at(int64_t row, int64_t nb, int64_t b) { return (row >> 5) * 32 * nb + b * 32 + (row & 31); }
+
 // ---------------------------------------------------------------------------
 // Kernel launchers (defined in k_quantize.hip, k_matvec.hip, k_gemm.hip).
 // Each checks the shapes its grid assumes and returns hipErrorInvalidValue
@@ -230,7 +244,7 @@ hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLay
 // weight type / shape has no GEMM (the matvec then serves m > 8 too).
 size_t gemm_workspace_bytes(int type, int64_t m, int64_t n, int64_t k);
 // The fewest rows for which launch_gemm is the faster path.
-int gemm_min_rows(int type);
+int gemm_min_rows(int type, int64_t k);
 // Workspace that lets launch_gemm_pair split its second weight as far as it would.
 size_t gemm_pair_workspace_bytes(int64_t m, int64_t n2, int64_t k);
 // y[e] = part[0][e] + part[1][e] + ... of `total` elements, in split order.
@@ -240,9 +254,6 @@ hipError_t launch_reduce(const float *part, float *y, int64_t total, int splits,
 size_t gemm8_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemm8(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, int64_t m, float *y, int32_t *S,
                         int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s);
-// Sums split-K partial tiles [tiles][splits][gbm][128] into y in split order.
-hipError_t launch_splitk_reduce(const float *part, float *y, int m, int n, int ntm, int gbm, int splits, int tiles,
-                                hipStream_t s);
 
 // The NIF crate's own kernels (k_crate.hip; shape_ops.rs).
 enum { CRATE_W_Q4_0 = 0, CRATE_W_I8 = 1, CRATE_W_F16 = 2 };

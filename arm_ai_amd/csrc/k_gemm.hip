@@ -58,14 +58,15 @@ struct Plan {
 //   512 x 14336 x 4096  128 x 256 tiles 78 us, 64 x 128 90
 //   512 x 5632 x 2048   64 x 128 28 us, 128 x 256 in two splits 33
 //   128 x 4096 x 4096   few rows 17.5 us, 64 x 128 in four splits 21.1
+//   512 x 2048 x 2048   32 x 128 tiles 18.9 us, 64 x 128 21.3, few rows 22.1
 //   16 x 14336 x 4096   few rows, four wavefronts 14.6 us, eight 17.7, 32 x 128 in four splits 16.3
 //   16 x 4096 x 14336   few rows, eight wavefronts in two splits 17.1 us, unsplit 19.0
 struct FormCost {
     float alone, full;
     int slots, blocks;
 };
-constexpr FormCost COST[] = {{1.3f, 0.82f, 2, 1},  {1.5f, 1.25f, 3, 1}, {4.3f, 4.3f, 1, 1},
-                             {2.85f, 2.28f, 2, 1}, {1.08f, 1.12f, 3, 4}, {1.93f, 3.0f, 1, 8}};
+constexpr FormCost COST[] = {{1.4f, 0.84f, 2, 1},  {1.7f, 1.27f, 3, 1}, {4.3f, 4.3f, 1, 1},
+                             {2.85f, 2.26f, 2, 1}, {1.3f, 1.4f, 3, 4},   {2.5f, 3.7f, 1, 8}};
 constexpr int NFORMS = 6;
 
 Plan kq_plan(int type, int64_t m, int64_t n, int64_t k) {
@@ -151,13 +152,21 @@ KqParams kq_params(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, i
 
 }  // namespace
 
-// Q5_K, Q2_K and Q3_K have no matrix-core matvec, and the dot4 matvec's time
-// grows with the rows: from three rows the GEMM's few-row forms are faster
-// (Q3_K 14336 x 4096: 2 rows 12.9 us against 15.3, 4 rows 20.4 against 15.3, 8
-// rows 35 against 15.4; 5632 x 2048: 7.4 against 8.8, 11.2 against 8.7, 18.8
-// against 8.7).  The matrix-core matvec keeps Q4_K and Q6_K up to its 8 rows
-// (11.0 against 14.1 at 8 x 14336 x 4096, 8.3 against 8.9 at 8 x 5632 x 2048).
-int gemm_min_rows(int type) { return type == TYPE_Q5_K || type == TYPE_Q2_K || type == TYPE_Q3_K ? 3 : 9; }
+// Q5_K, Q2_K, Q3_K and the Q8_0 family have no matrix-core matvec, and the
+// dot4 matvec's time grows with the rows: from three rows (four) the GEMM's
+// few-row forms are faster, as far as they take the row length.  Q3_K 14336 x
+// 4096: 2 rows 12.9 us against 15.3, 4 rows 20.4 against 15.3, 8 rows 35
+// against 15.4; 5632 x 2048: 7.4 against 8.8, 11.2 against 8.7, 18.8 against
+// 8.7.  Q8_0 14336 x 4096: 2 rows 15.0 us against 19.1, 4 rows 20.1 against
+// 19.1, 8 rows 30.3 against 18.8; 576 x 576: 6.2 against 8.1, 7.9 against 7.4,
+// 11.7 against 7.5.  The matrix-core matvec keeps Q4_K and Q6_K up to its 8
+// rows (11.0 against 14.1 at 8 x 14336 x 4096, 8.3 against 8.9 at 8 x 5632 x
+// 2048).
+int gemm_min_rows(int type, int64_t k) {
+    if (type == TYPE_Q8_0) return k <= 256 * (int64_t)Q8_FEW_MAX_GROUPS ? Q8_MIN_ROWS : 9;
+    if (type == TYPE_Q5_K || type == TYPE_Q2_K || type == TYPE_Q3_K) return k <= QK_K * (int64_t)KQ_FEW_MAX_NG ? 3 : 9;
+    return 9;
+}
 
 hipError_t launch_reduce(const float *part, float *y, int64_t total, int splits, hipStream_t s) {
     if (total % 4 == 0 && (((uintptr_t)y | (uintptr_t)part) & 15) == 0)

@@ -1,5 +1,5 @@
-// k_gemm8.hip -- prefill GEMM (m > 8) for Q8_0 weights on the int8 matrix
-// cores, gfx950.
+// k_gemm8.hip -- prefill GEMM for Q8_0 weights (and Q4_0 / Q5_0 on their
+// expanded copy) on the int8 matrix cores, gfx950.
 //
 // Replaces the M-row loop of candle-core 0.8.4 k_quants::matmul<BlockQ8_0>
 // at prefill (native/arm_ai_nif/src/llama_candle.rs:93; the activation is
@@ -20,26 +20,37 @@
 //   - acc = fma(t, d_x, acc): one rounding fewer than candle's mul-then-add
 //     (within the f32 tolerance of the output; the integer sums are bit-exact,
 //     see the dump variant).
+// 32 fmas against one MFMA of 32 cycles bind it to VALU issue whatever the
+// tile; what a form has to do is to keep two or three wavefronts per SIMD
+// issuing.
 //
-// Tiling.  A workgroup (4 wavefronts, two workgroups per CU) owns a 128 (m) x
-// 128 (n) tile; each wavefront a 64 x 64 block of four 32 x 32 MFMA tiles.
-// A step is 64 k-bytes (two blocks).  Per step, buffer loads into LDS copy:
-//   - the 128 activation rows' 64 quant bytes (16-byte chunks at position
-//     c ^ ((r >> 2) & 3) of the row, so 16 consecutive rows read
-//     conflict-free);
-//   - the 16 row blocks' four 128-byte weight lines (pieces 4s..4s+3 of group
-//     g = step / 4, s = step % 4), in their tile order [row block][piece][row];
-//   - d_x of both blocks for the 128 rows, gathered 4 bytes per lane into
-//     [block][row] order (four consecutive rows of a lane's MFMA output are
-//     then one 16-byte read);
-//   - the 128 columns' two f16 d_w (4 bytes of piece 16 of the group).
-// Four stages, issued three steps ahead.  Work items (tile, k-split) are
-// dealt so that all m-tiles and k-splits of one n-tile run on one XCD and
-// share its L2 copy of the weight rows.  Split-K partial tiles are summed in
-// split order by the Q4_K GEMM's reduce launch.
+// A lane's weight operand is a 16-byte piece of its own column (column l % 32,
+// half h = l / 32: piece 2 j + h of block j), loaded straight into registers
+// one group of eight blocks ahead, each again as soon as it is used.  The
+// activation comes from planes in the order of the MFMA operands
+// (q8_at, dt_at): a block of 32 rows is 1 KiB in lane order.
+//
+// Tiled form: a workgroup of four wavefronts owns 64 rows x 128 columns, each
+// wavefront 32 columns and all the rows; the activation of half a group (four
+// blocks) at a time goes global -> LDS by buffer-to-LDS copies, into two
+// stages, one half ahead; one s_waitcnt vmcnt and one barrier per half.  The
+// eight blocks of a group are summed apart and added to the output once: 2 %
+// more fmas' time, and the error against 64 bits stays below that of the
+// 128 x 128 tiles before (8.5e-8 against 9.6e-8 at 333 x 4096 x 4096, where one
+// chain over K had 1.5e-7); 240 VGPRs, two wavefronts per SIMD.
+// 333 x 4096 x 4096: 43.6 us before, 35.7 now; 512 x 14336 x 4096: 131.6, 105.8;
+// 512 x 5632 x 2048: 43.5, 31.6 (with the quantizer).
+// Few-row form (a tile of 32): the wavefronts of a workgroup share 32 columns
+// and take every fourth or eighth group each, with no stage and no barrier in
+// between, then add their sums through LDS in wavefront order.
+// Work items (tile, K split) are dealt so that the row tiles and splits of
+// one column tile run on one XCD; split-K partials are added in split order by
+// launch_reduce.
 #include "aq_internal.h"
 
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 namespace aq {
 
@@ -49,362 +60,398 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int G8T = 128;     // rows (m) and columns (n) per workgroup tile
-constexpr int G8K = 64;      // k-bytes per step: two Q8_0 blocks
-constexpr int G8NST = 4;     // stages in the LDS ring
 constexpr int G8XCD = 8;
-constexpr int TARGET_WG8 = 512;  // two workgroups per CU
-constexpr int G8COPIES = 6;      // copy instructions per wavefront and step
-constexpr int32_t C0 = 0x4B400000;   // bits of 1.5 * 2^23
-constexpr float C0F = 12582912.0f;   // 1.5 * 2^23
-
-struct L8 {
-    static constexpr int ACT = 0;                 // [128 rows][64 B], swizzled chunks
-    static constexpr int W = G8T * G8K;           // [16 row blocks][4 pieces][8 rows][16 B]
-    static constexpr int DX = 2 * G8T * G8K;      // [2 blocks][128 rows] f32
-    static constexpr int DW = DX + 2 * G8T * 4;   // [128 columns] two f16
-    static constexpr int PAD = DW + G8T * 4;      // landing area of the unused gather lanes
-    static constexpr int STAGE = PAD + 2 * 256;
-};
-static_assert(L8::STAGE * G8NST * 2 <= 160 * 1024, "two workgroups per CU");
+constexpr int32_t C0 = 0x4B400000;  // bits of 1.5 * 2^23
+constexpr float C0F = 12582912.0f;  // 1.5 * 2^23
+constexpr int PIECES = 17;          // of a group: 2 j, 2 j + 1 the quants of block j, 16 the eight f16 d
 
 struct Gemm8Params {
-    const uint8_t *w;      // row-block tiles
+    const uint8_t *w;   // row-block tiles
     int64_t rb_stride;
-    int ng;                // groups (8 blocks) per weight row
-    const int8_t *xq;      // [m][k] quants
-    const float *xd;       // [m][k/32] d_x
-    float *y;              // [m][n]
-    float *part;           // split-K partial tiles
-    int32_t *S, *Smin;     // integer dump [m][n][k/32] (DUMP only)
-    int m, n, k, nb;       // nb = k / 32
-    int ntm, tiles, splits, kss, items, per_xcd;  // kss: steps per split
+    int ng, nb;         // groups and blocks (k / 32) per row
+    const uint8_t *q8;  // activation quants (q8_at)
+    const float *dt;    // activation d (dt_at)
+    float *y;           // [m][n], or with splits > 1 the partials [splits][m][n]
+    int32_t *S, *Smin;  // integer dump [m][n][k/32] (DUMP only)
+    int m, n, k;
+    int ntm, splits, kgs, items, per_xcd;  // kgs: groups per split
 };
 
-template <bool DUMP>
-__global__ __launch_bounds__(256, 2) void gemm_q80_kernel(const Gemm8Params p) {
-    __shared__ __align__(16) uint8_t lds[G8NST * L8::STAGE];
-    const int xcd = blockIdx.x % G8XCD, local = blockIdx.x / G8XCD;
-    const int item = xcd * p.per_xcd + local;
-    if (local >= p.per_xcd || item >= p.items) return;  // uniform over the workgroup
-    const int tile = item / p.splits, split = item - tile * p.splits;
-    const int tn = tile / p.ntm, tm = tile - tn * p.ntm;
-    const int m0 = tm * G8T, n0 = tn * G8T;
-    const int nk = (p.nb + 1) / 2;  // steps over the whole row
-    const int ks0 = split * p.kss, ks1 = min(nk, ks0 + p.kss);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1, h = lane >> 5, l32 = lane & 31;
-    const int k = p.k;
-
-    const rsrc_t ra = buf_rsrc(p.xq, (uint32_t)((int64_t)p.m * k));
-    const rsrc_t rdx = buf_rsrc(p.xd, (uint32_t)((int64_t)p.m * p.nb * 4));
-    const int rb0 = n0 / 8, rb_all = (p.n + 7) / 8;
-    const int rb_here = min(G8T / 8, rb_all - rb0);
-    const rsrc_t rw = buf_rsrc(p.w + (int64_t)rb0 * p.rb_stride, (uint32_t)(rb_here * p.rb_stride));
-
-    // Per-lane offsets (fixed over the steps; the step enters as the scalar
-    // offset).  Copy instruction i of this wavefront, q = 2 * wave + i:
-    //   activations: LDS chunk t = 64q + lane -> row t/4, position t%4,
-    //                holding the row's chunk (t%4) ^ ((row >> 2) & 3);
-    //   weights:     row blocks 2q, 2q+1; lane -> (row block 2q + lane/32,
-    //                piece (lane%32)/8, row lane%8), 16 bytes;
-    //   gathers:     q 0..3 -> d_x of block q/2, rows 64(q%2) + lane;
-    //                q 4, 5 -> d_w pair of columns 64(q-4) + lane;
-    //                q 6, 7 -> unused (read out of range into the pad).
-    uint32_t aoff[2], woff[2], goff[2];
+__device__ __forceinline__ u32x4 ld16(const rsrc_t &r, uint32_t voff, int soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+}
+__device__ __forceinline__ v16i offset_acc() {
+    v16i c;
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int q = 2 * wave + i;
-        const int t = 64 * q + lane, r = t >> 2, cp = t & 3;
-        const int64_t ao = (int64_t)(m0 + r) * k + 16 * (cp ^ ((r >> 2) & 3));
-        aoff[i] = m0 + r < p.m ? (uint32_t)ao : BUF_OOB;  // rows past m read zeros
-        woff[i] = (uint32_t)((int64_t)(2 * q + (lane >> 5)) * p.rb_stride + (lane & 31) * 16);
-        if (q < 4) {
-            const int row = m0 + 64 * (q & 1) + lane;
-            goff[i] = (uint32_t)(((int64_t)row * p.nb + (q >> 1)) * 4);
-        } else if (q < 6) {
-            const int c = 64 * (q - 4) + lane;
-            goff[i] = (uint32_t)((int64_t)(c >> 3) * p.rb_stride + 16 * 128 + (c & 7) * 16);
-        } else {
-            goff[i] = BUF_OOB;
-        }
+    for (int r = 0; r < 16; r++) {
+        int v = C0;
+        asm volatile("" : "+v"(v));  // held in registers, not rebuilt for each MFMA
+        c[r] = v;
     }
-    uint8_t *const gdst0 = lds + (2 * wave < 4 ? L8::DX + 256 * (2 * wave) : 2 * wave < 6 ? L8::DW + 256 * (2 * wave - 4)
-                                                                                          : L8::PAD);
-    auto issue = [&](int slot_ks) {
-        // stage slot_ks % 4 gets step slot_ks's data; a step past the row's
-        // last (issued ahead, never read) reloads the last step, so no copy
-        // addresses memory past the rows
-        uint8_t *st = lds + (slot_ks & (G8NST - 1)) * L8::STAGE;
-        const int ks = min(slot_ks, nk - 1);
-        const int g = ks >> 2, s = ks & 3;
-        const int wsoff = (g * 17 + 4 * s) * 128;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int q = 2 * wave + i;
-            buf_to_lds16(ra, st + L8::ACT + 1024 * q, aoff[i], ks * G8K);
-            buf_to_lds16(rw, st + L8::W + 1024 * q, woff[i], wsoff);
-        }
-        // the two gathers: wave 0 -> d_x block 0 (both row halves), wave 1 ->
-        // d_x block 1, wave 2 -> d_w, wave 3 -> pad
-        const int gsoff = wave < 2 ? ks * 8 : wave < 3 ? g * 17 * 128 + 4 * s : 0;
-        buf_to_lds4(wave < 2 ? rdx : rw, st + (gdst0 - lds), goff[0], gsoff);
-        buf_to_lds4(wave < 2 ? rdx : rw, st + (gdst0 - lds) + 256, goff[1], gsoff);
-    };
-    auto afrag = [&](const uint8_t *st, int R, int s2) {  // 16 k-bytes of activation row R, block s2, half h
-        const int C = 2 * s2 + h;
-        return *(const v4i *)(st + L8::ACT + R * G8K + 16 * (C ^ ((R >> 2) & 3)));
-    };
-    auto bfrag = [&](const uint8_t *st, int Cn, int s2) {  // 16 k-bytes of weight row Cn, block s2, half h
-        const int piece = 2 * s2 + h;
-        return *(const v4i *)(st + L8::W + ((Cn >> 3) * 4 + piece) * 128 + (Cn & 7) * 16);
-    };
+    return c;
+}
+__device__ __forceinline__ uint32_t half_of(const u32x4 &d, int j) { return d[j >> 1] >> (16 * (j & 1)); }
 
-    v16i c0;
-#pragma unroll
-    for (int r = 0; r < 16; r++) c0[r] = C0;
-    float acc[2][2][16];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    // The copies are issued even for the steps a split never reaches (their
-    // data is not read), so every wavefront's vmcnt stays exact.
-    issue(ks0);
-    issue(ks0 + 1);
-    issue(ks0 + 2);
-    for (int ks = ks0; ks < ks1; ks++) {
-        wait_vmcnt<2 * G8COPIES>();  // this step's copies have landed (two later steps' may be in flight)
-        stage_barrier();             // ... for every wavefront; and step ks - 1's stage is free
-        issue(ks + 3);
-        const uint8_t *st = lds + (ks & (G8NST - 1)) * L8::STAGE;
-#pragma unroll
-        for (int s2 = 0; s2 < 2; s2++) {
-            const int blk = 2 * ks + s2;
-            if (blk >= p.nb) break;  // k an odd number of blocks: the last step's second block is padding
-            v4i af[2], bf[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                af[t] = afrag(st, 64 * wm + 32 * t + l32, s2);
-                bf[t] = bfrag(st, 64 * wn + 32 * t + l32, s2);
-            }
-            v16i D[2][2];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) D[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], c0, 0, 0, 0);
-            float dw[2], ndw[2];
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const uint32_t pr = *(const uint32_t *)(st + L8::DW + 4 * (64 * wn + 32 * j + l32));
-                dw[j] = f16_bits_to_f32(s2 ? pr >> 16 : pr & 0xffff);
-                ndw[j] = -C0F * dw[j];
-            }
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                float dx[16];
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const v4f v = *(const v4f *)(st + L8::DX + s2 * (G8T * 4) + 4 * (64 * wm + 32 * i + 8 * q + 4 * h));
-                    dx[4 * q] = v.x;
-                    dx[4 * q + 1] = v.y;
-                    dx[4 * q + 2] = v.z;
-                    dx[4 * q + 3] = v.w;
-                }
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const float t = __builtin_fmaf(u32_as_f32((uint32_t)D[i][j][r]), dw[j], ndw[j]);
-                        acc[i][j][r] = __builtin_fmaf(t, dx[r], acc[i][j][r]);
-                    }
-            }
-            if (DUMP) {
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int j = 0; j < 2; j++) {
-                        const int col = n0 + 64 * wn + 32 * j + l32;
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int row = m0 + 64 * wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                            if (row < p.m && col < p.n) {
-                                const int64_t o = ((int64_t)row * p.n + col) * p.nb + blk;
-                                p.S[o] = D[i][j][r] - C0;
-                                p.Smin[o] = 0;
-                            }
-                        }
-                    }
-            }
-        }
-    }
-    wait_vmcnt<0>();  // no copy may still be landing when the workgroup ends
-
-    if (p.splits == 1) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int col = n0 + 64 * wn + 32 * j + l32;
-            if (col >= p.n) continue;
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int row = m0 + 64 * wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (row < p.m) p.y[(int64_t)row * p.n + col] = acc[i][j][r];
-                }
-        }
-        return;
-    }
-    // split-K: this partial tile, [128 rows][128 columns], summed by the reduce launch
-    float *mine = p.part + ((int64_t)tile * p.splits + split) * (G8T * G8T);
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-                mine[(64 * wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3)) * G8T + 64 * wn + 32 * j + l32] = acc[i][j][r];
+// d_w of block j as f32, converted once: left to the compiler the conversion
+// goes into every fma as v_fma_mix_f32 (3 % slower at 512 x 4096 x 4096).
+__device__ __forceinline__ float dw_of(const u32x4 &d, int j) {
+    float f = f16_bits_to_f32(half_of(d, j));
+    asm volatile("" : "+v"(f));
+    return f;
 }
 
+// y += (S * d_w) * d_x (first: =) for the 16 outputs of a lane; dx: d_x of its rows.
+__device__ __forceinline__ void combine(float (&y)[16], const v16i &D, float dw, const v4f (&dx)[4], bool first = false) {
+    const float ndw = -C0F * dw;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const float t = __builtin_fmaf(u32_as_f32((uint32_t)D[r]), dw, ndw);
+        y[r] = first ? t * dx[r >> 2][r & 3] : __builtin_fmaf(t, dx[r >> 2][r & 3], y[r]);
+    }
+}
+
+struct Item {
+    int tile_n, m0, split;
+    bool ok;
+};
+__device__ __forceinline__ Item item_of(const Gemm8Params &p, int rows) {
+    const int xcd = (int)blockIdx.x % G8XCD, local = (int)blockIdx.x / G8XCD;
+    const int item = xcd * p.per_xcd + local;
+    const int tile = item / p.splits, tn = tile / p.ntm;
+    return {tn, rows * (tile - tn * p.ntm), item - tile * p.splits, local < p.per_xcd && item < p.items};
+}
+
+// ------------------------------------------------------------ tiled form
+template <int MT>
+struct L8 {  // two stages, one per half of a group
+    static constexpr int QS = MT * 4 * 1024;  // [row tile][4 blocks][lane] 16 bytes
+    static constexpr int DX = QS;             // [row tile][4 blocks][32 rows] f32
+    static constexpr int STAGE = QS + 1024;
+};
+
+template <int MT>
+__global__ __launch_bounds__(256, 2) void gemm8_kernel(Gemm8Params p) {
+    constexpr int NW = 4;
+    using L = L8<MT>;
+    __shared__ __align__(16) uint8_t lds[2 * L::STAGE];
+    const Item it = item_of(p, 32 * MT);
+    if (!it.ok) return;  // uniform over the workgroup
+    const int m0 = it.m0, tn = it.tile_n;
+    const int g0 = it.split * p.kgs, nit = min(p.ng, g0 + p.kgs) - g0;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, l32 = lane & 31;
+    const int nb = p.nb;
+
+    // activation copies: MT of the stage's 4 MT fragments per wave, of one row
+    // tile; d of the workgroup's rows (each wave the same).  Rows past m read
+    // zeros (quants) or what the plane's padding holds (d: of rows that are
+    // never stored); blocks past the row read zeros.
+    const rsrc_t rq = buf_rsrc(p.q8, (uint32_t)((int64_t)p.m * p.k));
+    const int mt32 = (p.m + 31) / 32;
+    const rsrc_t rd = buf_rsrc(p.dt, (uint32_t)((int64_t)mt32 * 128 * nb));
+    const rsrc_t rnone = buf_rsrc(p.q8, 0u);
+    const int ct = MT * wave / 4;  // the copied row tile
+    const int trow = m0 + 32 * ct, trows = min(32, p.m - trow);
+    const uint32_t qoff = l32 < trows ? (uint32_t)(trow * p.k + l32 * 32 + 16 * h) : BUF_OOB;
+    const int qblk = 32 * max(trows, 0);
+    static_assert(MT == 2);
+    const uint32_t doff = (uint32_t)(((m0 / 32 + h) * nb + (l32 >> 3)) * 128 + (lane & 7) * 16);  // row tile h
+    const bool d_ok = m0 / 32 + h < mt32;
+
+    const int nrb = (p.n + RB - 1) / RB, rb0 = 16 * tn, rb_here = min(16, nrb - rb0);
+    const rsrc_t rw = buf_rsrc(p.w + (int64_t)rb0 * p.rb_stride, (uint32_t)(rb_here * p.rb_stride));
+    const uint32_t woff = (uint32_t)((4 * wave + (l32 >> 3)) * p.rb_stride + (l32 & 7) * 16);
+
+    auto issue = [&](int i, auto HALF) {  // that half of group g0 + i
+        constexpr int HF = decltype(HALF)::value;
+        uint8_t *st = lds + HF * L::STAGE;
+        const int b0 = (g0 + i) * 8 + 4 * HF;
+#pragma unroll
+        for (int c = 0; c < MT; c++) {
+            const int f = MT * wave + c, b = b0 + f % 4;
+            buf_to_lds16(i < nit && b < nb ? rq : rnone, st + 1024 * f, qoff, b * qblk);
+        }
+        buf_to_lds16(i < nit ? rd : rnone, st + L::DX, d_ok && b0 + (l32 >> 3) < nb ? doff : BUF_OOB, b0 * 128);
+    };
+
+    float y[MT][16];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) y[t][r] = 0.0f;
+    const v16i c0 = offset_acc();
+    u32x4 q[8], dn;
+    auto load_q = [&](const rsrc_t &r, int j, int g) { q[j] = ld16(r, woff + 128u * h, (g * PIECES + 2 * j) * 128); };
+
+    issue(0, std::integral_constant<int, 0>{});
+    dn = ld16(rw, woff, (g0 * PIECES + 16) * 128);
+    __builtin_amdgcn_sched_barrier(0);  // (the loop's order, so that its waits count the same loads)
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        load_q(rw, j, g0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int i = 0; i < nit; i++) {
+        const rsrc_t r4 = i + 1 < nit ? rw : rnone;
+        u32x4 d = dn;
+        float gsum[MT][16];  // of the group: eight-term chains, then one term a group
+        auto half = [&](auto HALF) {
+            constexpr int HF = decltype(HALF)::value;
+            // this wave's copies of the half have landed (the weight loads
+            // issued since may stay in flight), then every wave's; and every
+            // wave has read the other stage
+            wait_vmcnt<HF == 0 ? 4 : 5>();
+            stage_barrier();
+            issue(HF == 0 ? i : i + 1, std::integral_constant<int, 1 - HF>{});
+            if constexpr (HF == 0) dn = ld16(r4, woff, ((g0 + i + 1) * PIECES + 16) * 128);
+            const uint8_t *st = lds + HF * L::STAGE;
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) {
+                const int j = 4 * HF + jj;
+                const float dw = dw_of(d, j);
+                v16i D[MT];
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    D[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*(const v4i *)(st + (4 * t + jj) * 1024 + 16 * lane),
+                                                                __builtin_bit_cast(v4i, q[j]), c0, 0, 0, 0);
+                load_q(r4, j, g0 + i + 1);
+#pragma unroll
+                for (int t = 0; t < MT; t++) {
+                    v4f dx[4];
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; g4++) dx[g4] = *(const v4f *)(st + L::DX + (4 * t + jj) * 128 + 4 * (8 * g4 + 4 * h));
+                    combine(gsum[t], D[t], dw, dx, j == 0);
+                }
+            }
+        };
+        half(std::integral_constant<int, 0>{});
+        half(std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) y[t][r] += gsum[t][r];
+    }
+    wait_vmcnt<0>();  // copies issued past the last group still write LDS
+
+    float *out = p.y + (p.splits > 1 ? (int64_t)it.split * p.m * p.n : 0);
+    const int col = 128 * tn + 32 * wave + l32;
+    if (col >= p.n) return;
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int row = m0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (row < p.m) out[(int64_t)row * p.n + col] = y[t][r];
+        }
+}
+
+// ------------------------------------------------------------ few rows
+// DUMP: the integer sums of every block instead of the outputs.
+template <int NW, bool DUMP>
+__global__ __launch_bounds__(64 * NW, 2) void few8_kernel(Gemm8Params p) {
+    extern __shared__ __align__(16) uint8_t dyn[];  // [NW][32][32] f32, then d [block][32 rows] f32
+    float *red = (float *)dyn;
+    float *dx = (float *)(dyn + NW * 4096);
+    const Item it = item_of(p, 32);
+    if (!it.ok) return;  // uniform over the workgroup
+    const int m0 = it.m0, tn = it.tile_n, rows = min(32, p.m - m0);
+    const int g0 = it.split * p.kgs, g1 = min(p.ng, g0 + p.kgs);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, l32 = lane & 31;
+    const int nb = p.nb;
+
+    const rsrc_t rq = buf_rsrc(p.q8, (uint32_t)((int64_t)p.m * p.k));
+    const rsrc_t rnone = buf_rsrc(p.q8, 0u);
+    const uint32_t qoff = l32 < rows ? (uint32_t)(m0 * p.k + l32 * 32 + 16 * h) : BUF_OOB;
+    const int qblk = 32 * rows;
+    const int nrb = (p.n + RB - 1) / RB, rb0 = 4 * tn, rb_here = min(4, nrb - rb0);
+    const rsrc_t rw = buf_rsrc(p.w + (int64_t)rb0 * p.rb_stride, (uint32_t)(rb_here * p.rb_stride));
+    const uint32_t woff = (uint32_t)((l32 >> 3) * p.rb_stride + (l32 & 7) * 16);
+
+    u32x4 q[8], a[8], dn;
+    int g = g0 + wave;
+    auto load = [&](int j, int gg, bool live) {
+        q[j] = ld16(live ? rw : rnone, woff + 128u * h, (gg * PIECES + 2 * j) * 128);
+        a[j] = ld16(live && gg * 8 + j < nb ? rq : rnone, qoff, (gg * 8 + j) * qblk);
+    };
+    dn = ld16(g < g1 ? rw : rnone, woff, (g * PIECES + 16) * 128);
+#pragma unroll
+    for (int j = 0; j < 8; j++) load(j, g, g < g1);
+    for (int e = tid; e < 256 * (g1 - g0); e += 64 * NW) {  // blocks past the row: zeros
+        const int b = 8 * g0 + (e >> 5), r = e & 31;
+        dx[e] = b < nb && r < rows ? p.dt[(int64_t)(m0 / 32) * 32 * nb + b * 32 + r] : 0.0f;
+    }
+    lds_barrier();
+
+    float y[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) y[r] = 0.0f;
+    const v16i c0 = offset_acc();
+    for (; g < g1; g += NW) {  // uniform over the wavefront
+        const bool more = g + NW < g1;
+        const u32x4 d = dn;
+        dn = ld16(more ? rw : rnone, woff, ((g + NW) * PIECES + 16) * 128);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, a[j]), __builtin_bit_cast(v4i, q[j]), c0, 0, 0, 0);
+            load(j, g + NW, more);
+            v4f dx4[4];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++) dx4[g4] = *(const v4f *)(dx + 256 * (g - g0) + 32 * j + 8 * g4 + 4 * h);
+            combine(y, D, dw_of(d, j), dx4);
+            if constexpr (DUMP) {
+                const int b = 8 * g + j, col = 32 * tn + l32;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int row = 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (row < rows && col < p.n && b < nb) {
+                        const int64_t o = ((int64_t)(m0 + row) * p.n + col) * nb + b;
+                        p.S[o] = D[r] - C0;
+                        p.Smin[o] = 0;
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (DUMP) return;
+
+    // red [wavefront][row of 32][column of 32]
+#pragma unroll
+    for (int r = 0; r < 16; r++) red[(wave * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * 32 + l32] = y[r];
+    lds_barrier();
+    float *out = p.y + (p.splits > 1 ? (int64_t)it.split * p.m * p.n : 0);
+    for (int e = tid; e < 32 * rows; e += 64 * NW) {
+        const int r = e >> 5, col = 32 * tn + (e & 31);
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) sum += red[w * 1024 + e];
+        if (col < p.n) out[(int64_t)(m0 + r) * p.n + col] = sum;
+    }
+}
+
+// ------------------------------------------------------------ plan
 struct Gemm8Plan {
-    int ntm, ntn, tiles, splits, kss;
+    int form, ntm, ntn, splits, kgs;  // form 0: 64 x 128; 1, 2: few rows, 4 or 8 wavefronts
     size_t ws;
 };
 
-// Split K (halves, quarters, ...) while there are fewer work items than two
-// per CU, each split keeping at least four steps.
+// The form and K split of least estimated time, as kq_plan's (k_gemm.hip):
+// the time of one step (a group, or one group per wavefront) of a workgroup
+// alone on its CU, its share when the CU holds more, the workgroups a CU
+// holds.  Measured over 576..14336 columns, K of 576..14336, 4..512 rows,
+// with the quantizer launch (the 128 x 128 tiles with four K splits before):
+//   16 x 4096 x 4096    few rows, eight wavefronts 11.4 us, four 14.9 (23.3)
+//   128 x 4096 x 4096   few rows, four wavefronts 18.2 us, eight 19.6, 64 x 128 in four splits 23.2 (26.2)
+//   333 x 4096 x 4096   64 x 128 in four splits 32.4 us, in two 36.4 (39.5)
+//   512 x 14336 x 4096  64 x 128 101.9 us, in two splits 104 (125)
+// (the 64 x 128 figures without the group sums, which add 2 %).
+struct FormCost {
+    int rows, cols;
+    float alone, full;
+    int slots, groups;
+};
+constexpr FormCost COST[] = {{64, 128, 2.4f, 1.45f, 3, 1}, {32, 32, 2.4f, 1.5f, 3, 4}, {32, 32, 3.0f, 3.5f, 1, 8}};
+
 Gemm8Plan gemm8_plan(int64_t m, int64_t n, int64_t k) {
-    Gemm8Plan g;
-    const int nk = (int)((k / QK8_0 + 1) / 2);
-    g.ntm = (int)((m + G8T - 1) / G8T);
-    g.ntn = (int)((n + G8T - 1) / G8T);
-    g.tiles = g.ntm * g.ntn;
-    g.splits = 1;
-    while ((int64_t)g.tiles * g.splits < TARGET_WG8 && nk / (2 * g.splits) >= 4) g.splits *= 2;
-    g.kss = (nk + g.splits - 1) / g.splits;
-    g.splits = (nk + g.kss - 1) / g.kss;
-    g.ws = g.splits > 1 ? (size_t)g.tiles * g.splits * G8T * G8T * 4 : 0;
-    return g;
+    const int ng = (int)((k / QK8_0 + 7) / 8);
+    const int most_splits = m <= 8 ? 1 : 16;  // up to 8 rows no split: those calls never needed a workspace
+    Gemm8Plan best{};
+    float best_us = 0.0f;
+    for (int form = 0; form < 3; form++) {
+        const FormCost &t = COST[form];
+        const int64_t ntm = (m + t.rows - 1) / t.rows, ntn = (n + t.cols - 1) / t.cols;
+        for (int splits = 1; splits <= most_splits && splits * 2 <= std::max(ng, 2); splits *= 2) {
+            const int kgs = (ng + splits - 1) / splits, ns = (ng + kgs - 1) / kgs;
+            if (form && kgs > Q8_FEW_MAX_GROUPS) continue;
+            const float c = (float)((ntm * ntn * ns + 255) / 256);  // workgroups of the busiest CU
+            const float step = c <= 1.0f ? t.alone : std::max(t.alone * std::ceil(c / t.slots), t.full * c);
+            const float us = ((kgs + t.groups - 1) / t.groups) * step + (ns > 1 ? 2.5f + 8.0f * ns * (float)m * (float)n / 3.5e6f : 0.0f);
+            if (best_us == 0.0f || us < best_us) {
+                best_us = us;
+                best = {form, (int)ntm, (int)ntn, ns, kgs, ns > 1 ? (size_t)ns * m * n * 4 : 0};
+            }
+        }
+    }
+    return best;
 }
 
 // Rows per launch: the copies address the activation quants with 32-bit
 // offsets (rows * k < 2^31); longer inputs run as several launches.
 int64_t gemm8_chunk_rows(int64_t m, int64_t k) {
-    const int64_t cap = (((int64_t)1 << 31) - 1) / k / G8T * G8T;
+    const int64_t cap = (((int64_t)1 << 31) - 1) / k / 128 * 128;
     return m < cap ? m : cap;
-}
-
-// y = sum over splits (in split order) of the partial tiles; one thread per
-// output element of a tile row.  A kernel boundary, not a fence, makes the
-// partials visible: a device-scope fence per workgroup costs an L2
-// write-back on this GPU.
-// V consecutive columns of one tile row per thread (V = 4: 16-byte loads and
-// stores, where n % 4 == 0 and y is 16-byte aligned, so that the four stay in
-// one output row; the partial tiles are 128 columns wide).  Indices in 32
-// bits: the launcher checks that the tiles' elements fit.  The sum starts
-// from 0 and adds the parts in order, whatever V.
-template <int V>
-__global__ __launch_bounds__(256) void gemm_splitk_reduce(const float *__restrict__ part, float *__restrict__ y, int m,
-                                                          int n, int ntm, int gbm, int splits, int tiles) {
-    const int per_tile = gbm * G8T;
-    const int e = ((int)blockIdx.x * 256 + (int)threadIdx.x) * V;
-    if (e >= tiles * per_tile) return;
-    const int tile = e / per_tile;
-    const int w = e - tile * per_tile;
-    const int tn = tile / ntm, tm = tile - tn * ntm;
-    const int row = tm * gbm + w / G8T, c = tn * G8T + w % G8T;
-    if (row >= m || c >= n) return;
-    const float *src = part + (int64_t)tile * splits * per_tile + w;
-    float *dst = y + (int64_t)row * n + c;
-    if (V == 4 && c + 4 <= n) {
-        float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (int s2 = 0; s2 < splits; s2++) {
-            const float4 t = *(const float4 *)(src + (int64_t)s2 * per_tile);
-            acc.x += t.x;
-            acc.y += t.y;
-            acc.z += t.z;
-            acc.w += t.w;
-        }
-        *(float4 *)dst = acc;
-    } else {
-        for (int j = 0; j < V && c + j < n; j++) {
-            float acc = 0.0f;
-            for (int s2 = 0; s2 < splits; s2++) acc += src[(int64_t)s2 * per_tile + j];
-            dst[j] = acc;
-        }
-    }
 }
 
 }  // namespace
 
-hipError_t launch_splitk_reduce(const float *part, float *y, int m, int n, int ntm, int gbm, int splits, int tiles,
-                                hipStream_t s) {
-    const int64_t elems = (int64_t)tiles * gbm * G8T;
-    if (elems + 4 * 256 > 0x7fffffff) return hipErrorInvalidValue;
-    if (n % 4 == 0 && (((uintptr_t)y | (uintptr_t)part) & 15) == 0)
-        gemm_splitk_reduce<4><<<(unsigned)((elems / 4 + 255) / 256), 256, 0, s>>>(part, y, m, n, ntm, gbm, splits, tiles);
-    else
-        gemm_splitk_reduce<1><<<(unsigned)((elems + 255) / 256), 256, 0, s>>>(part, y, m, n, ntm, gbm, splits, tiles);
-    return hipGetLastError();
-}
-
 size_t gemm8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-    if (m <= 0 || n <= 0 || k <= 0 || k % QK8_0 || k > (1 << 24)) return (size_t)-1;
+    if (m < Q8_MIN_ROWS || n <= 0 || k <= 0 || k % QK8_0 || k > (1 << 24)) return (size_t)-1;
     const int64_t mc = gemm8_chunk_rows(m, k);
     if (mc <= 0) return (size_t)-1;
     const Gemm8Plan g = gemm8_plan(mc, n, k);
-    if (g.tiles > GEMM_MAX_TILES) return (size_t)-1;
+    if ((int64_t)g.ntm * g.ntn > GEMM_MAX_TILES) return (size_t)-1;
     size_t ws = g.ws;
-    if (m % mc) ws = std::max(ws, gemm8_plan(m % mc, n, k).ws);  // the last, shorter launch
+    if (m % mc) ws = std::max(ws, gemm8_plan(m % mc, n, k).ws);
     return ws;
 }
 
 hipError_t launch_gemm8(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, int64_t m, float *y, int32_t *S,
                         int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s) {
     if (w.type != TYPE_Q8_0) return hipErrorNotSupported;
-    if (!w.slab || !y || !x.qs || !x.d || m <= 0 || n <= 0 || k <= 0 || k % QK8_0) return hipErrorInvalidValue;
-    if (m > 0x7fffffff || n > 0x7fffffff || k > (1 << 24) || w.ng != groups_of(TYPE_Q8_0, k)) return hipErrorInvalidValue;
+    if (!w.slab || !y || !x.q16 || m < Q8_MIN_ROWS || n <= 0 || k <= 0 || k % QK8_0) return hipErrorInvalidValue;
+    if (m > 0x7fffffff || n > 0x7fffffff || k > (1 << 24) || w.ng != (k / QK8_0 + 7) / 8) return hipErrorInvalidValue;
+    if ((int64_t)16 * w.rb_stride >= ((int64_t)1 << 31)) return hipErrorNotSupported;
     if ((S == nullptr) != (Smin == nullptr)) return hipErrorInvalidValue;
-    // one n-tile's weights, addressed with 32-bit offsets
-    if ((int64_t)(G8T / 8) * w.rb_stride >= ((int64_t)1 << 31)) return hipErrorNotSupported;
     const int64_t mc = gemm8_chunk_rows(m, k);
-    const int nb = (int)(k / QK8_0);
+    if (mc <= 0) return hipErrorNotSupported;
+    const int64_t nb = k / QK8_0;
     for (int64_t r0 = 0; r0 < m; r0 += mc) {
         const int64_t mm = std::min(mc, m - r0);
-        const Gemm8Plan g = gemm8_plan(mm, n, k);
-        if (g.tiles > GEMM_MAX_TILES) return hipErrorNotSupported;
-        if (g.splits > 1 && (!ws || ws_bytes < g.ws)) return hipErrorInvalidValue;
+        Gemm8Plan g = gemm8_plan(mm, n, k);
+        if (S) {  // the dump's form: few rows, split as far as d in LDS asks
+            g = {1, (int)((mm + 31) / 32), (int)((n + 31) / 32), (w.ng + Q8_FEW_MAX_GROUPS - 1) / Q8_FEW_MAX_GROUPS, 0, 0};
+            g.kgs = (w.ng + g.splits - 1) / g.splits;
+        }
+        if ((int64_t)g.ntm * g.ntn > GEMM_MAX_TILES) return hipErrorNotSupported;
+        if (g.ws && (!ws || ws_bytes < g.ws)) return hipErrorInvalidValue;
         Gemm8Params p;
         p.w = w.slab;
         p.rb_stride = w.rb_stride;
         p.ng = w.ng;
-        p.xq = x.qs + r0 * k;
-        p.xd = x.d + r0 * nb;
-        p.y = y + r0 * n;
-        p.part = (float *)ws;
+        p.nb = (int)nb;
+        p.q8 = (const uint8_t *)x.q16 + r0 * k;
+        p.dt = dt_plane(x, k) + r0 * nb;
+        p.y = g.splits > 1 ? (float *)ws : y + r0 * n;
         p.S = S ? S + r0 * n * nb : nullptr;
         p.Smin = Smin ? Smin + r0 * n * nb : nullptr;
         p.m = (int)mm;
         p.n = (int)n;
         p.k = (int)k;
-        p.nb = nb;
         p.ntm = g.ntm;
-        p.tiles = g.tiles;
         p.splits = g.splits;
-        p.kss = g.kss;
-        p.items = g.tiles * g.splits;
+        p.kgs = g.kgs;
+        p.items = g.ntm * g.ntn * g.splits;
         p.per_xcd = (p.items + G8XCD - 1) / G8XCD;
         const unsigned grid = (unsigned)(p.per_xcd * G8XCD);
-        if (S) gemm_q80_kernel<true><<<grid, 256, 0, s>>>(p);
-        else gemm_q80_kernel<false><<<grid, 256, 0, s>>>(p);
+        if (g.form == 0) gemm8_kernel<2><<<grid, 256, 0, s>>>(p);
+        else {
+            const int nw = g.form == 1 ? 4 : 8, lds = nw * 4096 + 1024 * p.kgs;
+            if (lds > 65536) {  // past what a launch may take unasked
+                const void *f = S         ? (const void *)few8_kernel<4, true>
+                                : nw == 4 ? (const void *)few8_kernel<4, false>
+                                          : (const void *)few8_kernel<8, false>;
+                const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+                if (e != hipSuccess) return e;
+            }
+            if (S) few8_kernel<4, true><<<grid, 256, lds, s>>>(p);
+            else if (nw == 4) few8_kernel<4, false><<<grid, 256, lds, s>>>(p);
+            else few8_kernel<8, false><<<grid, 512, lds, s>>>(p);
+        }
         hipError_t e = hipGetLastError();
+        if (e == hipSuccess && g.splits > 1 && !S) e = launch_reduce((const float *)ws, y + r0 * n, mm * n, g.splits, s);
         if (e != hipSuccess) return e;
-        if (g.splits > 1 && (e = launch_splitk_reduce(p.part, p.y, p.m, p.n, g.ntm, G8T, g.splits, g.tiles, s)) != hipSuccess)
-            return e;
     }
     return hipSuccess;
 }

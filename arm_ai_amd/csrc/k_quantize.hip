@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float *__restri
 
 // Eight lanes per 32-element block, 32 blocks per workgroup.
 template <bool VEC>
-__global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restrict__ x, int64_t nblocks,
+__global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restrict__ x, int64_t nblocks, int64_t k,
                                                             ActPlanes a) {
     const int64_t gb = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
     const int sub = threadIdx.x & 7;
@@ -68,6 +68,12 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restr
         a.d16[gb] = h;
         a.d[gb] = f16_bits_to_f32(h);
     }
+    if (a.q16 && a.m >= Q8_MIN_ROWS) {  // the GEMM's planes
+        const uint32_t nb = (uint32_t)(k / QK8_0);
+        const int64_t row = nblocks <= 0x7fffffff ? (uint32_t)gb / nb : gb / nb, b = gb - row * nb;
+        *(uint32_t *)((uint8_t *)a.q16 + q8_at(row, a.m, k, b) + 4 * sub) = packed;
+        if (sub == 0) dt_plane(a, k)[dt_at(row, nb, b)] = f16_bits_to_f32(h);
+    }
 }
 
 hipError_t launch_quantize_q8k(const float *x, int64_t m, int64_t k, ActPlanes a, hipStream_t s) {
@@ -90,9 +96,9 @@ hipError_t launch_quantize_q8_0(const float *x, int64_t m, int64_t k, ActPlanes 
     const int64_t grid = (nblocks + 31) / 32;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     if (((uintptr_t)x & 15) == 0)
-        quantize_q8_0_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
+        quantize_q8_0_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
     else
-        quantize_q8_0_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, a);
+        quantize_q8_0_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, s>>>(x, nblocks, k, a);
     return hipGetLastError();
 }
 

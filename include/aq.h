@@ -22,9 +22,9 @@
  *  - Weight type ids are GGUF/GGML dtype ids (Q4_0 = 2, Q5_0 = 6, Q8_0 = 8,
  *    Q2_K = 10, Q3_K = 11, Q4_K = 12, Q5_K = 13, Q6_K = 14).  Every type
  *    runs a matvec at m = 1 and small batches, and a prefill GEMM for more
- *    rows (m > 8; Q5_K, Q2_K and Q3_K m > 2; Q4_0 and Q5_0 on an int8 copy
- *    that the upload expands into the Q8_0 layout, 34 bytes per 32 weights
- *    beside their 18- or 22-byte decode tiles).
+ *    rows (m > 8; Q5_K, Q2_K and Q3_K m > 2, Q8_0, Q4_0 and Q5_0 m > 3; Q4_0
+ *    and Q5_0 on an int8 copy that the upload expands into the Q8_0 layout,
+ *    34 bytes per 32 weights beside their 18- or 22-byte decode tiles).
  *  - A weight is n rows (output features) by k columns (input features),
  *    row-major blocks, exactly candle's QTensor storage of shape (n, k).
  *  - Host-pointer entry points are synchronous at return.  Device-pointer

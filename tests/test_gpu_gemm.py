@@ -1,5 +1,5 @@
-"""The K-quant prefill GEMM (m > 8) at the edges of its tiles, K splits and
-value ranges, against the oracle: block sums bit-exact, outputs within the
+"""The prefill GEMMs at the edges of their tiles, K splits and value ranges,
+against the oracle: block sums bit-exact, outputs within the
 tolerance of an f32 sum in another order (tests/_metrics.py)."""
 import numpy as np
 import pytest
@@ -61,3 +61,18 @@ def test_extreme_sums(ctx, t):
     x[1] = 1.0
     x[2, ::3] = 0.5
     check_matmul(ctx, W, x, cond=False)
+
+
+# the Q8_0 GEMM and its few-row forms: rows of padded groups (k not a multiple
+# of 256), idle wavefronts, row tiles of one row, more than 64 KiB of d in LDS
+@pytest.mark.parametrize("t", [S.TYPE_Q8_0, S.TYPE_Q4_0, S.TYPE_Q5_0])
+@pytest.mark.parametrize("n,k,m", [(33, 96, 4), (576, 576, 5), (1000, 2304, 8), (130, 1312, 33), (100, 14336, 7),
+                                   (257, 1056, 65), (1536, 4096, 97), (520, 32, 200)])
+def test_q8_rows(ctx, t, n, k, m):
+    rng = np.random.default_rng(n + m)
+    check_matmul(ctx, S.make_weight(t, n, k, rng=rng), S.make_activation(m, k, seed=m + 2))
+
+
+def test_q8_large_tiles(ctx):
+    rng = np.random.default_rng(9)
+    check_matmul(ctx, S.make_weight(S.TYPE_Q8_0, 5000, 864, rng=rng), S.make_activation(500, 864, seed=1), sums=False, cond=False)
