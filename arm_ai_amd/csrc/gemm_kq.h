@@ -490,13 +490,13 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
     auto super_block = [&](int i) {
         // This wave's copies of the half have landed (those of the other half
         // were issued before; the weight loads stay in flight, the compiler
-        // waits for those where they are used), a barrier (every wave's
-        // copies have landed, and every wave has read the other half's stage,
-        // which the copies issued now overwrite).
+        // waits for those where they are used) and its LDS reads are done, a
+        // barrier (every wave's copies have landed, and every wave has read the
+        // other half's stage, which the copies issued now overwrite).
         auto enter = [&](auto HALF) {
             constexpr int HF = decltype(HALF)::value;
             wait_vmcnt<HF == 0 ? PIECES1 : HEADS + PIECES0>();
-            stage_barrier();
+            lds_barrier();
             issue(HF == 0 ? i : i + 1, std::integral_constant<int, 1 - HF>{});
         };
         enter(std::integral_constant<int, 0>{});

@@ -236,7 +236,7 @@ __global__ __launch_bounds__(256, 2) void int8_gemm_kernel(const int8_t *__restr
     issue(2);
     for (int ks = 0; ks < nk; ks++) {
         wait_vmcnt<2 * I8COPIES>();  // this step's copies have landed (two later steps' may be in flight)
-        stage_barrier();             // ... for every wavefront; and step ks - 1's stage is free
+        lds_barrier();               // ... for every wavefront; and step ks - 1's stage has been read
         issue(ks + 3);
         const uint8_t *st = lds + (ks & (I8NST - 1)) * I8STAGE;
 #pragma unroll

@@ -199,10 +199,10 @@ __global__ __launch_bounds__(256, 2) void gemm8_kernel(Gemm8Params p) {
         auto half = [&](auto HALF) {
             constexpr int HF = decltype(HALF)::value;
             // this wave's copies of the half have landed (the weight loads
-            // issued since may stay in flight), then every wave's; and every
-            // wave has read the other stage
+            // issued since may stay in flight) and its reads of the other stage
+            // are done, then every wave's
             wait_vmcnt<HF == 0 ? 4 : 5>();
-            stage_barrier();
+            lds_barrier();
             issue(HF == 0 ? i : i + 1, std::integral_constant<int, 1 - HF>{});
             if constexpr (HF == 0) dn = ld16(r4, woff, ((g0 + i + 1) * PIECES + 16) * 128);
             const uint8_t *st = lds + HF * L::STAGE;
