@@ -39,8 +39,12 @@ struct aq_ctx {
     float *attn_part = nullptr;
     // the output head's per-workgroup (largest logit, row) pairs
     int2 *head_part = nullptr;
+    // the prompt attention's split K and V (grow-only, for its calls alone)
+    void *attn_planes = nullptr;
+    size_t attn_planes_bytes = 0;
 };
 constexpr size_t ATTN_PART_BYTES = (size_t)2 << 20;
+constexpr size_t ATTN_PLANES_MAX = (size_t)2 << 30;
 constexpr int HEAD_PARTS = 4096;
 
 // Scratch of aq_qmatmul_f32_device_noalloc: a fixed array in the library's
@@ -155,6 +159,34 @@ int ensure_scratch(aq_ctx *c, size_t bytes) {
     c->scratch = p;
     c->scratch_bytes = want;
     return AQ_OK;
+}
+
+// The workspace of the prompt attention on the f16 matrix cores, or null: the
+// attention then runs without one.  Never under capture (a captured graph would
+// keep the address of a buffer that a later call may replace), nor past 2 GiB;
+// powers of two, so that prompts fed in chunks seldom replace it.
+void *attn_planes_of(aq_ctx *c, size_t bytes) {
+    if (bytes > ATTN_PLANES_MAX) return nullptr;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (bytes <= c->attn_planes_bytes) return c->attn_planes;
+    size_t want = (size_t)1 << 20;
+    while (want < bytes) want *= 2;
+    // another thread's capture does not forbid this thread's allocation
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (c->attn_planes && hipStreamSynchronize(c->stream) == hipSuccess) {
+        (void)hipFree(c->attn_planes);
+        c->attn_planes = nullptr;
+        c->attn_planes_bytes = 0;
+    }
+    if (!c->attn_planes && hipMalloc(&c->attn_planes, want) == hipSuccess) c->attn_planes_bytes = want;
+    (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return bytes <= c->attn_planes_bytes ? c->attn_planes : nullptr;
 }
 
 int ensure_pinned(aq_ctx *c, size_t bytes) {
@@ -321,6 +353,7 @@ int aq_ctx_destroy(aq_ctx *c) {
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->attn_part) (void)hipFree(c->attn_part);
     if (c->head_part) (void)hipFree(c->head_part);
+    if (c->attn_planes) (void)hipFree(c->attn_planes);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return AQ_OK;
@@ -1053,8 +1086,16 @@ int aq_llama_attn_prefill(aq_ctx *ctx, const float *d_q, int64_t ldq, const floa
     if (m == 0) return AQ_OK;
     int rc = use_device(ctx->device);
     if (rc) return rc;
-    const hipError_t e = launch_attn_prefill(d_q, ldq, d_k, ldk, d_v, ldv, d_cos, d_sin, index_pos, m, d_kcache,
-                                             d_vcache, n_head, n_kv, head_dim, max_seq, d_out, ctx->stream);
+    hipError_t e = check_attn_prefill(d_q, ldq, d_k, ldk, d_v, ldv, d_cos, d_sin, index_pos, m, d_kcache, d_vcache,
+                                      n_head, n_kv, head_dim, max_seq, d_out);
+    if (e == hipSuccess) {
+        void *ws = attn_planes_of(ctx, attn_prompt_workspace_bytes(index_pos + m, n_kv, head_dim));
+        e = launch_attn_prompt(d_q, ldq, d_k, ldk, d_v, ldv, d_cos, d_sin, index_pos, m, d_kcache, d_vcache, n_head, n_kv,
+                               head_dim, max_seq, d_out, ws, ws ? ctx->attn_planes_bytes : 0, ctx->stream);
+        if (e == hipErrorNotSupported)
+            e = launch_attn_prefill(d_q, ldq, d_k, ldk, d_v, ldv, d_cos, d_sin, index_pos, m, d_kcache, d_vcache, n_head,
+                                    n_kv, head_dim, max_seq, d_out, ctx->stream);
+    }
     if (e == hipErrorNotSupported) return fail(AQ_ERR_SHAPE, "head_dim %lld: the prompt attention takes 64 or 128", (long long)head_dim);
     return hip_status(e, "attn_prefill");
 }

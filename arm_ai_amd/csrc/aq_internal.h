@@ -323,16 +323,29 @@ hipError_t launch_attn_decode(const float *qk, const float *v, const float *cosb
 // and a second launch that combines the slices (hipErrorNotSupported for
 // shapes it does not take: head_dim other than 64 or 128, more than 8 query
 // heads per kv head, a workspace too small), its slice count and
-// partial-record bytes, and the prompt's causal attention.
+// partial-record bytes.
 int attn_split_slices(int64_t n_kv, int64_t max_seq);
 size_t attn_split_workspace_bytes(int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq);
 hipError_t launch_attn_split(const float *qk, const float *v, const float *cosb, const float *sinb,
                              const int64_t *d_pos, float *kc, float *vc, int64_t n_head, int64_t n_kv, int64_t hd,
                              int64_t max_seq, float *out, float *part, size_t part_bytes, hipStream_t s);
+// The prompt's attention: its argument check, the kernel on the f32 matrix
+// cores, and the one on the f16 matrix cores (each operand split into two f16
+// values) with a workspace for the split K and V: hipErrorNotSupported when
+// that is null or too small (attn_prompt_workspace_bytes: (size_t)-1 where no
+// size would do) or the grid too large.  Both take checked arguments.
+hipError_t check_attn_prefill(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
+                              const float *cosb, const float *sinb, int64_t index_pos, int64_t m, const float *kc,
+                              const float *vc, int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, const float *out);
 hipError_t launch_attn_prefill(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
                                const float *cosb, const float *sinb, int64_t index_pos, int64_t m, float *kc,
                                float *vc, int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, float *out,
                                hipStream_t s);
+size_t attn_prompt_workspace_bytes(int64_t kend, int64_t n_kv, int64_t hd);
+hipError_t launch_attn_prompt(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
+                              const float *cosb, const float *sinb, int64_t index_pos, int64_t m, float *kc, float *vc,
+                              int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, float *out, void *ws,
+                              size_t ws_bytes, hipStream_t s);
 hipError_t launch_argmax(const float *x, int64_t n, int64_t *d_tok, int64_t *d_pos, int64_t *hist, int64_t hist_len,
                          hipStream_t s);
 // The greedy pick from per-workgroup (value bits, row) pairs (the first row

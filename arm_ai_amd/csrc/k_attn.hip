@@ -403,6 +403,10 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(const float *__restrict__ 
     }
 }
 
+// For prompts that end at few keys, and where there is no workspace for the
+// split operands of attn_prompt_kernel (k_attn_prompt.hip): under capture, or
+// past its largest size.
+//
 // 2) attn_prefill_kernel: one workgroup of four wavefronts per (query tile
 //    of 32 rows, query head), on the f32 matrix cores
 //    (v_mfma_f32_32x32x2f32: f32 products, f32 sums).  Wavefront w takes the
@@ -657,10 +661,9 @@ hipError_t launch_attn_split(const float *qk, const float *v, const float *cosb,
     return hipGetLastError();
 }
 
-hipError_t launch_attn_prefill(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
-                               const float *cosb, const float *sinb, int64_t index_pos, int64_t m, float *kc,
-                               float *vc, int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, float *out,
-                               hipStream_t s) {
+hipError_t check_attn_prefill(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
+                              const float *cosb, const float *sinb, int64_t index_pos, int64_t m, const float *kc,
+                              const float *vc, int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, const float *out) {
     if (!q || !k || !v || !cosb || !sinb || !kc || !vc || !out) return hipErrorInvalidValue;
     if (m <= 0 || index_pos < 0 || max_seq <= 0 || index_pos + m > max_seq || max_seq > 0x7fffffff ||
         n_head <= 0 || n_kv <= 0 || n_head % n_kv || n_head > 65535)
@@ -668,6 +671,13 @@ hipError_t launch_attn_prefill(const float *q, int64_t ldq, const float *k, int6
     if (hd != 64 && hd != 128) return hipErrorNotSupported;
     if (ldq < n_head * hd || ldk < n_kv * hd || ldv < n_kv * hd) return hipErrorInvalidValue;
     if (((uintptr_t)kc | (uintptr_t)vc | (uintptr_t)out) & 15) return hipErrorInvalidValue;
+    return hipSuccess;
+}
+
+hipError_t launch_attn_prefill(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
+                               const float *cosb, const float *sinb, int64_t index_pos, int64_t m, float *kc,
+                               float *vc, int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, float *out,
+                               hipStream_t s) {
     rope_kv_kernel<<<(unsigned)m, 256, 0, s>>>(k, ldk, v, ldv, cosb, sinb, (int)index_pos, (int)n_kv, (int)hd,
                                                (int)max_seq, kc, vc);
     const unsigned grid = (unsigned)(((m + PM_QT - 1) / PM_QT) * n_head);

@@ -308,3 +308,131 @@ def test_embed_rows_and_silu_mul_rows(env):
     lib.check(L.aq_llama_silu_mul_rows(ctx.handle, dg.data_ptr(), du.data_ptr(), n, m, n, o2.data_ptr()))
     ctx.synchronize()
     assert np.array_equal(o2.cpu().numpy(), got)
+
+
+def _prefill_call(torch, lib, ctx, n_head, n_kv, hd, index_pos, m, max_seq, qk, v, kc, vc, cos, sin):
+    """(out, kc, vc) after aq_llama_attn_prefill on host arrays."""
+    width = (n_head + n_kv) * hd
+    dqk, dv, dkc, dvc, dcos, dsin = (_dev(torch, a) for a in (qk, v, kc, vc, cos, sin))
+    out = torch.empty((m, n_head * hd), dtype=torch.float32, device="cuda:0")
+    torch.cuda.synchronize()
+    lib.check(lib.load().aq_llama_attn_prefill(
+        ctx.handle, dqk.data_ptr(), width, dqk.data_ptr() + 4 * n_head * hd, width, dv.data_ptr(), n_kv * hd,
+        dcos.data_ptr(), dsin.data_ptr(), index_pos, m, dkc.data_ptr(), dvc.data_ptr(), n_head, n_kv, hd, max_seq,
+        out.data_ptr()))
+    ctx.synchronize()
+    return out.cpu().numpy(), dkc.cpu().numpy(), dvc.cpu().numpy()
+
+
+# The split-operand kernel's forms and edges: each (wavefronts per unit and key
+# range), last tiles and blocks of one row and of 31, prompts that begin within a
+# block of cached keys, units that do not fill the last workgroup.
+@pytest.mark.parametrize(
+    "n_head,n_kv,hd,index_pos,m",
+    [(4, 1, 64, 0, 321), (3, 3, 64, 650, 1), (9, 3, 64, 95, 1001), (8, 2, 128, 0, 161), (6, 2, 128, 319, 31),
+     (32, 32, 64, 0, 321), (32, 4, 64, 33, 450), (32, 8, 128, 95, 330), (33, 11, 128, 0, 1281)],
+)
+@pytest.mark.parametrize("scaled", [False, True])
+def test_prefill_split_operands(env, n_head, n_kv, hd, index_pos, m, scaled):
+    torch, lib, ctx = env
+    rng = np.random.default_rng(m + hd + scaled)
+    max_seq = index_pos + m + 3
+    qk = rng.standard_normal((m, (n_head + n_kv) * hd)).astype(np.float32)
+    v = rng.standard_normal((m, n_kv * hd)).astype(np.float32)
+    kc = rng.standard_normal((n_kv, max_seq, hd)).astype(np.float32)
+    vc = rng.standard_normal((n_kv, max_seq, hd)).astype(np.float32)
+    if scaled:  # powers of two that change from block to block, and a block of zeros
+        pos = np.arange(max_seq)
+        ks, vs = 2.0 ** -(pos // 32 % 5), 2.0 ** (9 * (pos // 32 % 4) - 13)
+        ks[64:96] = vs[64:96] = 0.0
+        kc *= ks[None, :, None].astype(np.float32)
+        vc *= vs[None, :, None].astype(np.float32)
+        qk[:, n_head * hd:] *= ks[index_pos:index_pos + m, None].astype(np.float32)
+        v *= vs[index_pos:index_pos + m, None].astype(np.float32)
+        qk[:, :n_head * hd] *= (2.0 ** -(np.arange(m) % 9))[:, None].astype(np.float32)
+    cos, sin = _tables(hd, max_seq)
+    got, kc1, vc1 = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, index_pos, m, max_seq, qk, v, kc, vc, cos, sin)
+    want, kc2, vc2 = _prefill_ref(qk[:, :n_head * hd], qk[:, n_head * hd:], v, kc, vc, cos, sin, index_pos, n_head, n_kv, hd)
+    # |score error| <= sum |q k| / sqrt(hd) (2^-22 + hd / 16 2^-24): at most
+    # 7.3 * 7.2e-7 = 5.2e-6 for normal values and hd = 128, and as much relative in
+    # the output; the sums of the output add 2^-22 + 3 * keys / 16 2^-24
+    assert _rel(got, want) <= 1e-5
+    assert np.array_equal(kc1, kc2) and np.array_equal(vc1, vc2)
+
+
+# What the split cannot hold goes through plain f32: values beyond 2^50 or below
+# 2^-50, infinities and NaN, in K, V or a query row.
+@pytest.mark.parametrize("where,value", [("v", 2.0 ** 70), ("v", 2.0 ** -70), ("k", 2.0 ** -70), ("q", 2.0 ** -70),
+                                         ("q", 2.0 ** 70), ("v", np.nan), ("k", np.nan), ("v", np.inf), ("q", np.nan)])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_prefill_values_beyond_the_split(env, hd, where, value):
+    torch, lib, ctx = env
+    n_head, n_kv, m, at = 6, 2, 330, 201
+    rng = np.random.default_rng(hd)
+    qk = rng.standard_normal((m, (n_head + n_kv) * hd)).astype(np.float32)
+    v = rng.standard_normal((m, n_kv * hd)).astype(np.float32)
+    cos, sin = _tables(hd, m)
+    if where == "v":
+        v[192:224, hd:] *= value if np.isfinite(value) else 1
+        if not np.isfinite(value):
+            v[at, hd:] = value  # kv head 1, key 201
+    elif where == "k":
+        if np.isfinite(value):
+            qk[192:224, (n_head + 1) * hd:] *= value
+        else:
+            qk[at, (n_head + 1) * hd:] = value
+    elif np.isfinite(value):
+        qk[at, 4 * hd:5 * hd] *= value  # query head 4 (kv head 1), row 201
+        if value > 1:  # scores within the f32 range
+            qk[:, n_head * hd:] *= 2.0 ** -70
+    else:
+        qk[at, 4 * hd:5 * hd] = value
+    z = np.zeros((n_kv, m, hd), np.float32)
+    got, _, _ = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, m, m, qk, v, z, z, cos, sin)
+    with np.errstate(all="ignore"):
+        want, _, _ = _prefill_ref(qk[:, :n_head * hd], qk[:, n_head * hd:], v, z, z, cos, sin, 0, n_head, n_kv, hd)
+    got, want = got.reshape(m, n_head, hd), want.reshape(m, n_head, hd)
+    fine = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fine)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    for r0, r1 in ((0, 192), (192, 224), (224, m)):  # (apart: their sizes differ by 2^70)
+        for h in range(n_head):
+            f = fine[r0:r1, h]
+            if f.any():
+                assert _rel(got[r0:r1, h][f], want[r0:r1, h][f]) <= 1e-5
+
+
+def test_prefill_under_capture_is_the_f32_kernel(env):
+    """A captured prompt keeps no workspace address: its replays, after larger
+    prompts have grown the workspace, give the f32 kernel's result."""
+    torch, lib, ctx = env
+    L = lib.load()
+    n_head, n_kv, hd, m = 8, 2, 64, 400
+    rng = np.random.default_rng(3)
+    g = [rng.standard_normal(s).astype(np.float32) for s in ((m, (n_head + n_kv) * hd), (m, n_kv * hd))]
+    cos, sin = _tables(hd, m)
+    z = np.zeros((n_kv, m, hd), np.float32)
+    want, _, _ = _prefill_ref(g[0][:, :n_head * hd], g[0][:, n_head * hd:], g[1], z, z, cos, sin, 0, n_head, n_kv, hd)
+    dqk, dv, dkc, dvc, dcos, dsin = (_dev(torch, a) for a in (*g, z, z, cos, sin))
+    out = torch.empty((m, n_head * hd), dtype=torch.float32, device="cuda:0")
+    width = (n_head + n_kv) * hd
+    torch.cuda.synchronize()
+    handle = ctypes.c_void_p()
+    lib.check(L.aq_ctx_stream(ctx.handle, ctypes.byref(handle)))
+    stream = torch.cuda.ExternalStream(handle.value)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        lib.check(L.aq_llama_attn_prefill(
+            ctx.handle, dqk.data_ptr(), width, dqk.data_ptr() + 4 * n_head * hd, width, dv.data_ptr(), n_kv * hd,
+            dcos.data_ptr(), dsin.data_ptr(), 0, m, dkc.data_ptr(), dvc.data_ptr(), n_head, n_kv, hd, m, out.data_ptr()))
+    for n in (0, 700, 2100):  # eager prompts between the replays
+        if n:
+            c2, s2 = _tables(hd, n)
+            z2 = np.zeros((n_kv, n, hd), np.float32)
+            a = rng.standard_normal((n, width)).astype(np.float32)
+            _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, n, n, a, a[:, :n_kv * hd].copy(), z2, z2, c2, s2)
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _rel(out.cpu().numpy(), want) <= 1e-5
