@@ -68,10 +68,18 @@ struct FormCost {
 constexpr FormCost COST[] = {{1.4f, 0.84f, 2, 1},  {1.7f, 1.27f, 3, 1}, {4.3f, 4.3f, 1, 1},
                              {2.85f, 2.26f, 2, 1}, {1.3f, 1.4f, 3, 4},   {2.5f, 3.7f, 1, 8}};
 constexpr int NFORMS = 6;
+// The time of a step against Q4_K's.  A form of 32 rows builds the weight
+// operands for one row tile only, which costs most where they are two digits
+// (Q6_K): 512 x 2048 x 5632 takes 49.3 us in 32 x 128 tiles, 40.7 in 64 x 128 with
+// two splits; 512 x 4096 x 4096 57.6 and 49.0 us.
+constexpr float WEIGHT_Q6K[] = {1.8f, 1.42f, 1.3f, 1.3f, 1.3f, 1.3f};
+constexpr float WEIGHT_Q3K[] = {1.3f, 1.25f, 1.2f, 1.2f, 1.05f, 1.05f};
+float step_weight(int type, int form) {
+    return type == TYPE_Q6_K ? WEIGHT_Q6K[form] : type == TYPE_Q3_K ? WEIGHT_Q3K[form] : type == TYPE_Q5_K ? 1.1f : 1.0f;
+}
 
 Plan kq_plan(int type, int64_t m, int64_t n, int64_t k) {
     const int ng = (int)(k / QK_K);
-    const float weight = type == TYPE_Q6_K ? 1.4f : type == TYPE_Q5_K ? 1.1f : 1.0f;  // time of a step against Q4_K's
     // up to 8 rows no split: those calls never needed a workspace
     const int most_splits = m <= 8 ? 1 : 16;
     Plan best{};
@@ -86,7 +94,7 @@ Plan kq_plan(int type, int64_t m, int64_t n, int64_t k) {
             if (t.blocks > 1 && kbs > KQ_FEW_MAX_NG) continue;
             const float c = (float)((ntm * ntn * ns + 255) / 256);  // workgroups of the busiest CU
             const float step = c <= 1.0f ? t.alone : std::max(t.alone * std::ceil(c / t.slots), t.full * c);
-            const float us = weight * ((kbs + t.blocks - 1) / t.blocks) * step +
+            const float us = step_weight(type, form) * ((kbs + t.blocks - 1) / t.blocks) * step +
                              (ns > 1 ? 2.5f + 8.0f * ns * (float)m * (float)n / 3.5e6f : 0.0f);
             if (best_us == 0.0f || us < best_us) {
                 best_us = us;
