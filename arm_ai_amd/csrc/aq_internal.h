@@ -333,7 +333,7 @@ hipError_t launch_attn_split(const float *qk, const float *v, const float *cosb,
 // cores, and the one on the f16 matrix cores (each operand split into two f16
 // values) with a workspace for the split K and V: hipErrorNotSupported when
 // that is null or too small (attn_prompt_workspace_bytes: (size_t)-1 where no
-// size would do) or the grid too large.  Both take checked arguments.
+// size would do or the other kernel is faster) or the grid too large.  Both take checked arguments.
 hipError_t check_attn_prefill(const float *q, int64_t ldq, const float *k, int64_t ldk, const float *v, int64_t ldv,
                               const float *cosb, const float *sinb, int64_t index_pos, int64_t m, const float *kc,
                               const float *vc, int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, const float *out);

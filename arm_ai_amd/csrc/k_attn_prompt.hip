@@ -557,6 +557,11 @@ hipError_t run(const Prompt &p, hipStream_t s) {
 }  // namespace
 
 size_t attn_prompt_workspace_bytes(int64_t kend, int64_t n_kv, int64_t hd) {
+    // The split costs a pass over the keys and a longer start: 16 rows and 16
+    // keys of 32/4 heads of 64 take 9.1 us on the f32 cores, 10.4 here; 256 rows
+    // 13.6 and 13.7, 300 rows 17.3 and 15.5; of 32/8 heads of 128, 128 rows 17.5
+    // and 17.5, 256 rows 24.5 and 21.5.
+    if (kend * hd <= 20480) return (size_t)-1;
     const int64_t nblk = (kend + KB - 1) / KB;
     if (nblk * 256 * hd >= ((int64_t)1 << 31)) return (size_t)-1;  // (32-bit offsets into a kv head's planes)
     return (size_t)(n_kv * nblk) * (size_t)(256 * hd + sizeof(int2));
@@ -583,11 +588,6 @@ hipError_t launch_attn_prompt(const float *q, int64_t ldq, const float *k, int64
                               const float *cosb, const float *sinb, int64_t index_pos, int64_t m, float *kc, float *vc,
                               int64_t n_head, int64_t n_kv, int64_t hd, int64_t max_seq, float *out, void *ws,
                               size_t ws_bytes, hipStream_t s) {
-    // The split costs a pass over the keys and a longer start: 16 rows and 16
-    // keys of 32/4 heads of 64 take 9.1 us on the f32 cores, 10.4 here; 256 rows
-    // 13.6 and 13.7, 300 rows 17.3 and 15.5; of 32/8 heads of 128, 128 rows 17.5
-    // and 17.5, 256 rows 24.5 and 21.5.
-    if ((index_pos + m) * hd <= 20480) return hipErrorNotSupported;
     if (attn_prompt_workspace_bytes(index_pos + m, n_kv, hd) > ws_bytes || !ws || n_kv > 65535) return hipErrorNotSupported;
     Prompt p{q, k, v, cosb, sinb, ldq, ldk, ldv, (int)index_pos, (int)m, (int)n_head, (int)n_kv, (int)max_seq,
              (int)((index_pos + m + KB - 1) / KB), kc, vc, (uint8_t *)ws, nullptr, out};
