@@ -498,6 +498,9 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
             wait_vmcnt<HF == 0 ? PIECES1 : HEADS + PIECES0>();
             lds_barrier();
             issue(HF == 0 ? i : i + 1, std::integral_constant<int, 1 - HF>{});
+            // the next wait counts the loads that follow: no copy may sink past one
+            // (the compiler moved d's behind the heads)
+            __builtin_amdgcn_sched_barrier(0);
         };
         enter(std::integral_constant<int, 0>{});
         v16f acc[MT][NT];
@@ -644,6 +647,7 @@ __device__ __forceinline__ void body(const KqParams &p, uint8_t *lds, int bid) {
     };
 
     issue(0, std::integral_constant<int, 0>{});
+    __builtin_amdgcn_sched_barrier(0);
     load_all<TYPE, NT>(v, rw, rwd, woff, doff, h, kb0);
     for (int i = 0; i < nit; i++) super_block(i);
     wait_vmcnt<0>();  // copies issued past the last super-block still write LDS
