@@ -19,7 +19,7 @@ import pytest
 from arm_ai_amd import build
 
 OBJDUMP = next((p for p in ("/opt/rocm/llvm/bin/llvm-objdump", shutil.which("llvm-objdump")) if p and os.path.exists(p)), None)
-NAMES = [b"kq6kernelI", b"pair_kernelI"]
+NAMES = [b"kq6kernelI", b"pair_kernelI", b"gemm8_kernelI"]
 DONE = 1 << 20  # no copy outstanding
 
 INSTR = re.compile(r"^\s+([a-z][a-z0-9_]+)(.*?)//\s*([0-9A-F]+):")
@@ -100,8 +100,8 @@ def kernels(tmp_path_factory):
     return funcs
 
 
-# the K-quant tiles of every type and the pair of two weights
-@pytest.mark.parametrize("name,least", [("2kq6kernelI", 25), ("2kq11pair_kernelI", 2)])
+# the K-quant tiles of every type, the pair of two weights, the Q8_0 tiles
+@pytest.mark.parametrize("name,least", [("2kq6kernelI", 25), ("2kq11pair_kernelI", 2), ("12gemm8_kernelI", 1)])
 def test_copies_are_waited_for(kernels, name, least):
     found = {n: c for n, c in kernels.items() if name in n}
     assert len(found) >= least
