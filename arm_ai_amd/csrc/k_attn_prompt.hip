@@ -13,10 +13,19 @@
 // (exact): a query row by its largest value, a block of 32 keys by the block's
 // (both to 2^14 .. 2^15), a block of 32 V rows to 2^11 .. 2^15 by a multiple
 // of 2^4, and the probabilities by 2^12.  The score scale takes up the first
-// two, the output sums are kept in units of the V block last added.  Where a
-// query row or a block has a largest value outside 2^-50 .. 2^50 (2^-40 ..
-// 2^40 for V) and not zero, or an infinity or NaN, the workgroups that would
-// read it go through attn_rows, in plain f32.
+// two, the output sums are kept in units of the V block last added.
+//
+// What does not fit goes through attn_rows, in plain f32, in the workgroups that
+// would read it:
+// - A query row or a block with a largest value outside 2^-50 .. 2^50 (2^-40 ..
+//   2^40 for V) and not zero, or with an infinity or NaN.
+// - A query row and a block of keys whose largest values have exponents that add
+//   to more than SCORE_EXP: a term of a score could pass 2^15.  f16 ends at 2^-39
+//   of a block's largest value, also for the rows far below it, and up to SCORE_EXP
+//   that is at most 2^-18 of a base-2 score for each operand (all dims at the worst;
+//   2^-24 for normal values beside one key of 2^15).  Scores stay below 2^23, so
+//   that their rounding (an exponent is one fma, its reference was rounded) adds at
+//   most 1/4 to an exponent, and a probability times 2^P_EXP stays an f16 number.
 //
 // 1) attn_planes_kernel: one workgroup per 32 keys and kv head rotates the
 //    prompt's k rows into the cache, copies its v rows there, and writes the
@@ -36,7 +45,8 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int KB = 32;                  // keys of a block, queries of a wavefront
-constexpr int BAD_EXP = INT_MIN;        // a block that f16 cannot hold
+constexpr int BAD_EXP = 1 << 20;        // a block that f16 cannot hold
+constexpr int SCORE_EXP = 16;           // most that the exponents of a query row and a K block add to
 constexpr int P_EXP = 12;               // probabilities are kept times 2^12
 constexpr float SLACK = 3.0f;           // ... and may exceed 1 by 2^SLACK (attn_prompt_kernel)
 
@@ -56,11 +66,11 @@ struct Prompt {
 
 __device__ __forceinline__ uint32_t mag(float x) { return f32_as_u32(x) & 0x7fffffffu; }
 
-// Exponent by which values of magnitude up to `bits` are divided.
+// Exponent by which values of magnitude up to `bits` are divided (zeros: the least).
 template <int LIMIT>
 __device__ __forceinline__ int scale_exp(uint32_t bits) {
     const int e = (int)(bits >> 23) - 127;
-    if (bits == 0) return 0;
+    if (bits == 0) return -LIMIT - 14;
     return e > LIMIT || e < -LIMIT ? BAD_EXP : e - 14;
 }
 
@@ -179,7 +189,7 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(Prompt p) {
     __syncthreads();
     top = max(max(smax[0], smax[1]), max(smax[2], smax[3]));
     int e = is_v ? scale_exp<40>(top) : scale_exp<50>(top);
-    if (is_v && e != BAD_EXP) e = (e + 3) & ~3;
+    if (is_v && e != BAD_EXP) e = top == 0 ? 0 : (e + 3) & ~3;
     if (tid == 0) *(is_v ? &ex->y : &ex->x) = e;
     if (e == BAD_EXP) return;  // uniform over the workgroup; the block's planes are not read
 
@@ -209,7 +219,8 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(Prompt p) {
 
 // The tile's rows in plain f32, where an operand does not fit the split: the
 // wavefronts take the rows in turn, a lane per key for the scores, the lanes
-// along the dims for the output.
+// along the dims for the output.  Every sum in four chains, as one of hd or of all
+// the keys rounds twice as far from 64 bits as attn_prefill_kernel does.
 template <int HD>
 __device__ void attn_rows(const Prompt &p, int h, int kvh, int qb, int rows, int first, int step, float *qs, float *ps) {
     const int lane = threadIdx.x & 63;
@@ -225,22 +236,22 @@ __device__ void attn_rows(const Prompt &p, int h, int kvh, int qb, int rows, int
             qs[2 * lane + 1] = a * sn + b * c;
         }
         __builtin_amdgcn_wave_barrier();
-        float mrun = -INFINITY, lrun = 0.0f, acc[HD / 64];
-        for (float &a : acc) a = 0.0f;
+        float mrun = -INFINITY, lrun = 0.0f, acc[HD / 64][4];
+        for (int i = 0; i < HD / 16; i++) acc[i / 4][i % 4] = 0.0f;
         for (int k0 = 0; k0 <= qpos; k0 += 64) {
             const int key = k0 + lane;
             float s = -INFINITY;
             if (key <= qpos) {
                 const float4 *kr = (const float4 *)(kh + (int64_t)key * HD);
-                s = 0.0f;
+                float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 for (int d = 0; d < HD / 4; d++) {
                     const float4 t = kr[d];
-                    s = __builtin_fmaf(t.x, qs[4 * d], s);
-                    s = __builtin_fmaf(t.y, qs[4 * d + 1], s);
-                    s = __builtin_fmaf(t.z, qs[4 * d + 2], s);
-                    s = __builtin_fmaf(t.w, qs[4 * d + 3], s);
+                    c.x = __builtin_fmaf(t.x, qs[4 * d], c.x);
+                    c.y = __builtin_fmaf(t.y, qs[4 * d + 1], c.y);
+                    c.z = __builtin_fmaf(t.z, qs[4 * d + 2], c.z);
+                    c.w = __builtin_fmaf(t.w, qs[4 * d + 3], c.w);
                 }
-                s *= sc2;
+                s = ((c.x + c.y) + (c.z + c.w)) * sc2;
             }
             float bm = s;
             for (int o = 1; o < 64; o *= 2) bm = fmaxf(bm, __shfl_xor(bm, o));
@@ -253,13 +264,18 @@ __device__ void attn_rows(const Prompt &p, int h, int kvh, int qb, int rows, int
             __builtin_amdgcn_wave_barrier();
             ps[lane] = e;
             __builtin_amdgcn_wave_barrier();
-            for (float &a : acc) a *= scale;
-            for (int kk = 0; kk < 64 && k0 + kk <= qpos; kk++)
-                for (int d = 0; d < HD / 64; d++)
-                    acc[d] = __builtin_fmaf(ps[kk], vh[(int64_t)(k0 + kk) * HD + 64 * d + lane], acc[d]);
+            for (int i = 0; i < HD / 16; i++) acc[i / 4][i % 4] *= scale;
+            for (int kk = 0; kk < 64 && k0 + kk <= qpos; kk += 4) {
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (k0 + kk + c <= qpos)
+                        for (int d = 0; d < HD / 64; d++)
+                            acc[d][c] = __builtin_fmaf(ps[kk + c], vh[(int64_t)(k0 + kk + c) * HD + 64 * d + lane], acc[d][c]);
+            }
         }
         for (int d = 0; d < HD / 64; d++)
-            p.out[(int64_t)(qb + r) * p.n_head * HD + (int64_t)h * HD + 64 * d + lane] = acc[d] / lrun;
+            p.out[(int64_t)(qb + r) * p.n_head * HD + (int64_t)h * HD + 64 * d + lane] =
+                ((acc[d][0] + acc[d][1]) + (acc[d][2] + acc[d][3])) / lrun;
         __builtin_amdgcn_wave_barrier();
     }
 }
@@ -347,7 +363,8 @@ __global__ __launch_bounds__(64 * QW * KG, 2) void attn_prompt_kernel(Prompt p) 
     const int eq = scale_exp<50>(qmax);
     const int2 *ex = p.exps + (int64_t)kvh * p.nblk;
     int bad = eq == BAD_EXP;
-    for (int b = tid; b < nkb; b += 64 * QW * KG) bad |= ex[b].x == BAD_EXP || ex[b].y == BAD_EXP;
+    const int eqm = scale_exp<50>(f32_as_u32(wave_max_f(u32_as_f32(qmax))));  // of the wavefront's rows
+    for (int b = lane; b < nkb; b += 64) bad |= ex[b].x + eqm > SCORE_EXP - 28 || ex[b].y == BAD_EXP;
     if (__syncthreads_or(bad)) {  // uniform; the copies in flight end before LDS is written again
         wait_vmcnt<0>();
         __syncthreads();

@@ -402,6 +402,96 @@ def test_prefill_values_beyond_the_split(env, hd, where, value):
                 assert _rel(got[r0:r1, h][f], want[r0:r1, h][f]) <= 1e-5
 
 
+def _prefill_captured(torch, lib, ctx, n_head, n_kv, hd, m, qk, v, cos, sin):
+    """out of a prompt at position 0 through the f32 kernel, which a captured call runs."""
+    width = (n_head + n_kv) * hd
+    z = np.zeros((n_kv, m, hd), np.float32)
+    dqk, dv, dkc, dvc, dcos, dsin = (_dev(torch, a) for a in (qk, v, z, z, cos, sin))
+    out = torch.empty((m, n_head * hd), dtype=torch.float32, device="cuda:0")
+    handle = ctypes.c_void_p()
+    lib.check(lib.load().aq_ctx_stream(ctx.handle, ctypes.byref(handle)))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.ExternalStream(handle.value)):
+        lib.check(lib.load().aq_llama_attn_prefill(
+            ctx.handle, dqk.data_ptr(), width, dqk.data_ptr() + 4 * n_head * hd, width, dv.data_ptr(), n_kv * hd,
+            dcos.data_ptr(), dsin.data_ptr(), 0, m, dkc.data_ptr(), dvc.data_ptr(), n_head, n_kv, hd, m, out.data_ptr()))
+    graph.replay()
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _scores(qk, kc, cos, sin, n_head):
+    """[m, n_head, key] of a prompt at position 0 in 64 bits, -inf past the row; kc: the cache after it."""
+    n_kv, m, hd = kc.shape
+    q = _rope(qk[:, :n_head * hd].reshape(m, n_head, hd), cos[:, None, :], sin[:, None, :]).astype(np.float64)
+    s = np.stack([q[:, h] @ kc[h * n_kv // n_head].astype(np.float64).T for h in range(n_head)], 1) / np.sqrt(hd)
+    return np.where(np.arange(m)[None, None] <= np.arange(m)[:, None, None], s, -np.inf)
+
+
+def _row_errors(got, want, m, n_head):
+    """Error of each row and head, relative to that row's largest output."""
+    got, want = (a.astype(np.float64).reshape(m, n_head, -1) for a in (got, want))
+    return np.abs(got - want).max(-1) / np.abs(want).max(-1)
+
+
+# Scores up to the split's limit and far past it.  A row whose two largest scores
+# lie closer than the rounding of a sum of that size (2^-18 of the largest, 64
+# roundings) may weigh them otherwise and is left out, but must be finite.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("scale", [5, 6, 7, 10, 13, 20, 40])
+def test_prefill_large_scores(env, hd, scale):
+    torch, lib, ctx = env
+    n_head, n_kv, m = 6, 2, 330
+    rng = np.random.default_rng(hd + scale)
+    qk = (2.0 ** scale * rng.standard_normal((m, (n_head + n_kv) * hd))).astype(np.float32)
+    qk[200, :n_head * hd] = 0.0  # a query of zeros: the mean of the values before it
+    v = rng.standard_normal((m, n_kv * hd)).astype(np.float32)
+    cos, sin = _tables(hd, m)
+    z = np.zeros((n_kv, m, hd), np.float32)
+    got, kc, _ = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, m, m, qk, v, z, z, cos, sin)
+    want, _, _ = _prefill_ref(qk[:, :n_head * hd], qk[:, n_head * hd:], v, z, z, cos, sin, 0, n_head, n_kv, hd)
+    assert np.isfinite(got).all()
+    s = _scores(qk, kc, cos, sin, n_head)
+    top = np.sort(s, -1)[..., -2:]
+    # 30: a second key of e^-30 changes nothing
+    clear = top[..., 1] - top[..., 0] > 30 + np.abs(s).max(-1, initial=0, where=np.isfinite(s)) * 2.0 ** -18
+    clear[200] = clear[0] = True
+    assert clear.mean() > (0.7 if scale > 5 else 0.5)
+    assert _row_errors(got, want, m, n_head)[clear].max() <= 2e-6
+
+
+# One key (31: the last of its block, which the rows before it do not see) far
+# above the others: every row as exact as the f32 kernel has it.  Left out are the
+# rows that weigh key 31 against others: a score of 2^exp is rounded, and one row
+# says nothing of how far.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("where", ["k"])
+@pytest.mark.parametrize("exp", [8, 13, 16, 20, 28, 38])
+def test_prefill_one_large_key(env, hd, where, exp):
+    torch, lib, ctx = env
+    n_head, n_kv, m = 6, 2, 330
+    rng = np.random.default_rng(hd + exp)
+    qk = rng.standard_normal((m, (n_head + n_kv) * hd)).astype(np.float32)
+    v = rng.standard_normal((m, n_kv * hd)).astype(np.float32)
+    (qk[:, n_head * hd:] if where == "k" else v)[31] *= 2.0 ** exp
+    cos, sin = _tables(hd, m)
+    z = np.zeros((n_kv, m, hd), np.float32)
+    got, kc, _ = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, m, m, qk, v, z, z, cos, sin)
+    f32 = _prefill_captured(torch, lib, ctx, n_head, n_kv, hd, m, qk, v, cos, sin)
+    want, _, _ = _prefill_ref(qk[:, :n_head * hd], qk[:, n_head * hd:], v, z, z, cos, sin, 0, n_head, n_kv, hd)
+    a, b = (_row_errors(o, want, m, n_head) for o in (got, f32))
+    clear = np.ones((m, n_head), bool)
+    if where == "k":
+        s = _scores(qk, kc, cos, sin, n_head)
+        rest = np.where(np.arange(m) == 31, -np.inf, s).max(-1)
+        clear[31:] = np.abs(s[31:, :, 31] - rest[31:]) > 30
+    for rows in (slice(0, 31), slice(31, m)):
+        c = clear[rows]
+        assert c.mean() > 0.7
+        assert a[rows][c].max() <= 1.5 * b[rows][c].max(), (rows, a[rows][c].max(), b[rows][c].max())
+
+
 def test_prefill_under_capture_is_the_f32_kernel(env):
     """A captured prompt keeps no workspace address: its replays, after larger
     prompts have grown the workspace, give the f32 kernel's result."""
