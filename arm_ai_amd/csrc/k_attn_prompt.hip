@@ -19,6 +19,9 @@
 // would read it:
 // - A query row or a block with a largest value outside 2^-50 .. 2^50 (2^-40 ..
 //   2^40 for V) and not zero, or with an infinity or NaN.
+// - A block of V with a row or a dim, not zero, whose largest value is below 2^-14
+//   of the block's.  f16 ends at 2^-36 of that (2^-40 where it lies high in its
+//   2^4), which is 2^-22 of the row's or the dim's: where 22 bits end as well.
 // - A query row and a block of keys whose largest values have exponents that add
 //   to more than SCORE_EXP: a term of a score could pass 2^15.  f16 ends at 2^-39
 //   of a block's largest value, also for the rows far below it, and up to SCORE_EXP
@@ -109,13 +112,34 @@ __device__ __forceinline__ float sum_halves(float v) {
     return u32_as_f32(r[0]) + u32_as_f32(r[1]);
 }
 
+// The largest of a over the lanes of a wavefront, for eight values a lane: those of
+// a[2 q] and a[2 q + 1] in the lanes of 16-lane row q.
+__device__ __forceinline__ void wave_max8(const uint32_t (&a)[8], uint32_t (&r)[2]) {
+    uint32_t h[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {  // lanes 0 .. 31: a[i], 32 .. 63: a[i + 4]
+        const auto t = __builtin_amdgcn_permlane32_swap(a[i], a[i + 4], false, false);
+        h[i] = max((uint32_t)t[0], (uint32_t)t[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {  // rows 0, 2: h[i], 1, 3: h[i + 2]
+        const auto t = __builtin_amdgcn_permlane16_swap(h[i], h[i + 2], false, false);
+        uint32_t v = max((uint32_t)t[0], (uint32_t)t[1]);
+        v = max(v, (uint32_t)dpp_i<DPP_QUAD_XOR1>((int)v));
+        v = max(v, (uint32_t)dpp_i<DPP_QUAD_XOR2>((int)v));
+        v = max(v, (uint32_t)dpp_i<DPP_HALF_MIRROR>((int)v));
+        r[i] = max(v, (uint32_t)dpp_i<DPP_ROW_MIRROR>((int)v));
+    }
+}
+
 // blockIdx.z 0: K, 1: V of the block.  Bound by latency, so every load is issued
 // before the first is used (keys past the end: the last one's, zeroed after).
 template <int HD>
 __global__ __launch_bounds__(256) void attn_planes_kernel(Prompt p) {
     constexpr int NP = HD / 64;  // pieces of eight values per thread
     __shared__ uint32_t smax[4];
-    __shared__ u32x4 img[2][HD * 4];  // K hi, lo
+    __shared__ u32x4 img[2][HD * 4];  // K hi, lo; V: the largest of each dim and key
+    uint32_t(*const dmax)[HD] = (uint32_t(*)[HD])img, (*const kmax)[32] = (uint32_t(*)[32])(dmax + 4);  // [eight keys], [64 dims]
     const int b = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, kend = p.index_pos + p.m;
     const bool is_v = blockIdx.z;
     int2 *const ex = p.exps + (int64_t)g * p.nblk + b;
@@ -179,8 +203,18 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(Prompt p) {
                 const int key = KB * b + 16 * st + 4 * hh + (e & 3) + 8 * (e >> 2);
                 if (key >= p.index_pos && key < kend) p.vc[((int64_t)g * p.max_seq + key) * HD + dim] = x[i][e];
                 if (key >= kend) x[i][e] = 0.0f;
-                top = max(top, mag(x[i][e]));
             }
+            uint32_t a[8], r[2], of_dim = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                a[e] = mag(x[i][e]);
+                of_dim = max(of_dim, a[e]);
+            }
+            top = max(top, of_dim);
+            dmax[2 * st + hh][dim] = of_dim;
+            wave_max8(a, r);
+            const int e = (tid & 63) >> 4 << 1;  // of a lane's row: values e and e + 1
+            if ((tid & 15) < 2) kmax[HD == 128 ? dim >> 6 : 0][16 * st + 4 * hh + (e & 3) + (tid & 15) + 8 * (e >> 2)] = r[tid & 1];
         }
     }
 #pragma unroll
@@ -189,7 +223,17 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(Prompt p) {
     __syncthreads();
     top = max(max(smax[0], smax[1]), max(smax[2], smax[3]));
     int e = is_v ? scale_exp<40>(top) : scale_exp<50>(top);
-    if (is_v && e != BAD_EXP) e = top == 0 ? 0 : (e + 3) & ~3;
+    if (is_v) {  // every wavefront looks at every dim and key: no second barrier
+        bool low = false;
+#pragma unroll
+        for (int i = tid & 63; i < HD + 32; i += 64) {
+            const uint32_t of = i < HD ? max(max(dmax[0][i], dmax[1][i]), max(dmax[2][i], dmax[3][i]))
+                                       : max(kmax[0][i - HD], HD == 128 ? kmax[1][i - HD] : 0u);
+            low |= of != 0 && u32_as_f32(of) < u32_as_f32(top) * 0x1p-14f;
+        }
+        if (__any(low)) e = BAD_EXP;
+        if (e != BAD_EXP) e = top == 0 ? 0 : (e + 3) & ~3;
+    }
     if (tid == 0) *(is_v ? &ex->y : &ex->x) = e;
     if (e == BAD_EXP) return;  // uniform over the workgroup; the block's planes are not read
 

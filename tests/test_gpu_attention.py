@@ -466,7 +466,7 @@ def test_prefill_large_scores(env, hd, scale):
 # rows that weigh key 31 against others: a score of 2^exp is rounded, and one row
 # says nothing of how far.
 @pytest.mark.parametrize("hd", [64, 128])
-@pytest.mark.parametrize("where", ["k"])
+@pytest.mark.parametrize("where", ["k", "v"])
 @pytest.mark.parametrize("exp", [8, 13, 16, 20, 28, 38])
 def test_prefill_one_large_key(env, hd, where, exp):
     torch, lib, ctx = env
@@ -490,6 +490,38 @@ def test_prefill_one_large_key(env, hd, where, exp):
         c = clear[rows]
         assert c.mean() > 0.7
         assert a[rows][c].max() <= 1.5 * b[rows][c].max(), (rows, a[rows][c].max(), b[rows][c].max())
+
+
+# The range inside a block of V: one key far above the others of its block, at each
+# place in it, and dims far below the others.  Each dim of the rows before that key
+# as exact as the f32 kernel has it (15: just past the range that the split takes,
+# 13: just inside it).
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("exp", [13, 15, 24])
+def test_prefill_range_of_v(env, hd, exp):
+    torch, lib, ctx = env
+    n_head, n_kv, m = 2, 1, 330
+    cos, sin = _tables(hd, m)
+    z = np.zeros((n_kv, m, hd), np.float32)
+    rng = np.random.default_rng(hd + exp)
+    qk = rng.standard_normal((m, (n_head + n_kv) * hd)).astype(np.float32)
+    v0 = rng.standard_normal((m, n_kv * hd)).astype(np.float32)
+    base, _, _ = _prefill_ref(qk[:, :n_head * hd], qk[:, n_head * hd:], v0, z, z, cos, sin, 0, n_head, n_kv, hd)
+    f32 = _prefill_captured(torch, lib, ctx, n_head, n_kv, hd, m, qk, v0, cos, sin)
+    err = np.abs(f32 - base).reshape(m, -1)
+    for at in range(96, 128):
+        v = v0.copy()
+        v[at] *= 2.0 ** exp
+        got, _, _ = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, m, m, qk, v, z, z, cos, sin)
+        # (the rows before key `at` do not see it)
+        assert np.abs(got - base)[:at].max() <= 1.5 * err.max(), at
+    for d in range(0, hd, 5):
+        v = v0.copy()
+        v[:, d] *= 2.0 ** -exp
+        got, _, _ = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, m, m, qk, v, z, z, cos, sin)
+        # (scaling by a power of two is exact: that dim's outputs scale with it)
+        own = got.reshape(m, n_head, hd)[..., d] * 2.0 ** exp
+        assert np.abs(own - base.reshape(m, n_head, hd)[..., d]).max() <= 1.5 * err.max(), d
 
 
 def test_prefill_under_capture_is_the_f32_kernel(env):
