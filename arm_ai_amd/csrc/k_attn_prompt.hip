@@ -15,10 +15,12 @@
 // of 2^4, and the probabilities by 2^12.  The score scale takes up the first
 // two, the output sums are kept in units of the V block last added.
 //
-// What does not fit goes through attn_rows, in plain f32, in the workgroups that
-// would read it:
+// What does not fit goes through plain f32, in the workgroups that would read it.
+// attn_rows takes:
 // - A query row or a block with a largest value outside 2^-50 .. 2^50 (2^-40 ..
 //   2^40 for V) and not zero, or with an infinity or NaN.
+// The f32 matrix cores (attn_f32: 2048 rows of 32/8 heads of 128 take 426 us, 391 in
+// attn_prefill_kernel, 6900 through attn_rows) take:
 // - A block of V with a row or a dim, not zero, whose largest value is below 2^-14
 //   of the block's.  f16 ends at 2^-36 of that (2^-40 where it lies high in its
 //   2^4), which is 2^-22 of the row's or the dim's: where 22 bits end as well.
@@ -48,7 +50,8 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int KB = 32;                  // keys of a block, queries of a wavefront
-constexpr int BAD_EXP = 1 << 20;        // a block that f16 cannot hold
+constexpr int BAD_EXP = 1 << 20;        // a block for attn_rows
+constexpr int WIDE_EXP = 1 << 19;       // a block of V for the f32 matrix cores
 constexpr int SCORE_EXP = 16;           // most that the exponents of a query row and a K block add to
 constexpr int P_EXP = 12;               // probabilities are kept times 2^12
 constexpr float SLACK = 3.0f;           // ... and may exceed 1 by 2^SLACK (attn_prompt_kernel)
@@ -231,11 +234,10 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(Prompt p) {
                                        : max(kmax[0][i - HD], HD == 128 ? kmax[1][i - HD] : 0u);
             low |= of != 0 && u32_as_f32(of) < u32_as_f32(top) * 0x1p-14f;
         }
-        if (__any(low)) e = BAD_EXP;
-        if (e != BAD_EXP) e = top == 0 ? 0 : (e + 3) & ~3;
+        if (e != BAD_EXP) e = __any(low) ? WIDE_EXP : top == 0 ? 0 : (e + 3) & ~3;
     }
     if (tid == 0) *(is_v ? &ex->y : &ex->x) = e;
-    if (e == BAD_EXP) return;  // uniform over the workgroup; the block's planes are not read
+    if (e >= WIDE_EXP) return;  // uniform over the workgroup; the block's planes are not read
 
 #pragma unroll
     for (int i = 0; i < NP; i++) {
@@ -324,6 +326,54 @@ __device__ void attn_rows(const Prompt &p, int h, int kvh, int qb, int rows, int
     }
 }
 
+// The key blocks first, first + step, .. of a unit on the f32 matrix cores, its
+// operands from the cache: the running max, sum and output (times 1).
+template <int HD>
+__device__ __forceinline__ void attn_f32(const Prompt &p, int kvh, int qb, int qpos, int first, int step, const float (&qx)[HD / 16][8],
+                                         float &mrun, float &lrun, v16f (&o)[HD / 32]) {
+    const int lane = threadIdx.x & 63, j = lane & 31, hh = lane >> 5, last = p.index_pos + p.m - 1;
+    const float *kh = p.kc + (int64_t)kvh * p.max_seq * HD, *vh = p.vc + (int64_t)kvh * p.max_seq * HD;
+    const float sc2 = 1.4426950408889634f / sqrtf((float)HD);
+    for (int k0 = first * KB; k0 <= min(last, p.index_pos + qb + KB - 1); k0 += step * KB) {
+        const float4 *kr = (const float4 *)(kh + (int64_t)min(k0 + j, last) * HD + 8 * hh);
+        v16f s[2];
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[0][r] = s[1][r] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < HD / 16; st++) {
+            const float4 a = kr[4 * st], b = kr[4 * st + 1];
+            const float kx[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[i], qx[st][i], s[i & 1], 0, 0, 0);
+        }
+        float x[16], bm = -INFINITY, sum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            x[r] = k0 + 8 * (r >> 2) + 4 * hh + (r & 3) > qpos ? -INFINITY : (s[0][r] + s[1][r]) * sc2;
+            bm = fmaxf(bm, x[r]);
+        }
+        const float mnew = fmaxf(mrun, max_halves(bm)), msafe = mnew == -INFINITY ? 0.0f : mnew;
+        const float scale = __builtin_amdgcn_exp2f(mrun - msafe);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            x[r] = __builtin_amdgcn_exp2f(x[r] - msafe);
+            sum += x[r];
+        }
+        lrun = __builtin_fmaf(lrun, scale, sum_halves(sum));
+        mrun = mnew;
+#pragma unroll
+        for (int b = 0; b < HD / 32; b++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[b][r] *= scale;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int key = min(k0 + 8 * (r >> 2) + 4 * hh + (r & 3), last);
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vh[(int64_t)key * HD + 32 * b + j], x[r], o[b], 0, 0, 0);
+            }
+        }
+    }
+}
+
 // 2) One workgroup of QW x KG wavefronts takes QW units of a kv head, a unit
 //    being 32 query rows of one of its query heads; KG wavefronts share a unit,
 //    wavefront group w taking the key blocks w, w + KG, ..., each with a running
@@ -406,25 +456,13 @@ __global__ __launch_bounds__(64 * QW * KG, 2) void attn_prompt_kernel(Prompt p) 
     qmax = max(qmax, (uint32_t)__shfl_xor((int)qmax, 32));
     const int eq = scale_exp<50>(qmax);
     const int2 *ex = p.exps + (int64_t)kvh * p.nblk;
-    int bad = eq == BAD_EXP;
+    int bad = eq == BAD_EXP, wide = bad;
     const int eqm = scale_exp<50>(f32_as_u32(wave_max_f(u32_as_f32(qmax))));  // of the wavefront's rows
-    for (int b = lane; b < nkb; b += 64) bad |= ex[b].x + eqm > SCORE_EXP - 28 || ex[b].y == BAD_EXP;
-    if (__syncthreads_or(bad)) {  // uniform; the copies in flight end before LDS is written again
-        wait_vmcnt<0>();
-        __syncthreads();
-        float *own = (float *)(lds + wave * 1024);
-        if (u0 + qw < units) attn_rows<HD>(p, h, kvh, qb, rows, kg, KG, own, own + HD);
-        return;
+    for (int b = lane; b < nkb; b += 64) {
+        const int2 e = ex[b];
+        bad |= max(e.x, e.y) == BAD_EXP;
+        wide |= e.x + eqm > SCORE_EXP - 28 || e.y >= WIDE_EXP;
     }
-    v8h qh[NS], ql[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) qx[s][i] = ldexpf(qx[s][i], -eq);
-        split8(qx[s], qh[s], ql[s]);
-    }
-
-    const float scq = ldexpf(1.4426950408889634f / sqrtf((float)HD), eq);  // log2(e) / sqrt(hd)
     float mrun = -INFINITY, lrun = 0.0f;
     int eo = 0;  // the output is in units of 2^eo
     v16f o[NB];
@@ -432,123 +470,142 @@ __global__ __launch_bounds__(64 * QW * KG, 2) void attn_prompt_kernel(Prompt p) 
     for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
+    if (__syncthreads_or(wide)) {  // uniform; the copies in flight end before LDS is written again
+        wait_vmcnt<0>();
+        if (__syncthreads_or(bad)) {
+            float *own = (float *)(lds + wave * 1024);
+            if (u0 + qw < units) attn_rows<HD>(p, h, kvh, qb, rows, kg, KG, own, own + HD);
+            return;
+        }
+        attn_f32<HD>(p, kvh, qb, qpos, kg, KG, qx, mrun, lrun, o);
+        eo = P_EXP;
+    } else {
+        v8h qh[NS], ql[NS];
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) qx[s][i] = ldexpf(qx[s][i], -eq);
+            split8(qx[s], qh[s], ql[s]);
+        }
 
-    v8h ph[2], pl[2];
-    // a block's exponents, loaded a block ahead: before the copies, so that
-    // waiting for them does not wait for those
-    int2 e, en = ex[min(kg, nkb - 1)];
-    auto next_exps = [&](int it) {
-        e = make_int2(__builtin_amdgcn_readfirstlane(en.x), __builtin_amdgcn_readfirstlane(en.y));
-        en = ex[min((it + 1) * KG + kg, nkb - 1)];
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    auto scores = [&](int blk, const uint8_t *kst) {
-        const int k0 = blk * KB;
-        v16f s;
-#pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = 0.0f;
-        // the small products first, then the large: one chain, K hi kept
-        v8h kh[NS], kl[2];
-        auto load = [&](int st) {
-            kl[st & 1] = *(const v8h *)(kst + 64 * HD + (st * 64 + lane) * 16);
-            kh[st] = *(const v8h *)(kst + (st * 64 + lane) * 16);
+        const float scq = ldexpf(1.4426950408889634f / sqrtf((float)HD), eq);  // log2(e) / sqrt(hd)
+        v8h ph[2], pl[2];
+        // a block's exponents, loaded a block ahead: before the copies, so that
+        // waiting for them does not wait for those
+        int2 e, en = ex[min(kg, nkb - 1)];
+        auto next_exps = [&](int it) {
+            e = make_int2(__builtin_amdgcn_readfirstlane(en.x), __builtin_amdgcn_readfirstlane(en.y));
+            en = ex[min((it + 1) * KG + kg, nkb - 1)];
+            __builtin_amdgcn_sched_barrier(0);
         };
-        load(0);
+        auto scores = [&](int blk, const uint8_t *kst) {
+            const int k0 = blk * KB;
+            v16f s;
 #pragma unroll
-        for (int st = 0; st < NS; st++) {
-            if (st + 1 < NS) load(st + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[st & 1], qh[st], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[st], ql[st], s, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+            for (int r = 0; r < 16; r++) s[r] = 0.0f;
+            // the small products first, then the large: one chain, K hi kept
+            v8h kh[NS], kl[2];
+            auto load = [&](int st) {
+                kl[st & 1] = *(const v8h *)(kst + 64 * HD + (st * 64 + lane) * 16);
+                kh[st] = *(const v8h *)(kst + (st * 64 + lane) * 16);
+            };
+            load(0);
 #pragma unroll
-        for (int st = 0; st < NS; st++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[st], qh[st], s, 0, 0, 0);
-        // lane (j, hh) register r: query j, key k0 + 8 (r / 4) + 4 hh + r % 4
-        if (k0 + KB - 1 > p.index_pos + qb) {  // the block holds keys past some row
+            for (int st = 0; st < NS; st++) {
+                if (st + 1 < NS) load(st + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[st & 1], qh[st], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[st], ql[st], s, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (k0 + 8 * (r >> 2) + 4 * hh + (r & 3) > qpos) s[r] = -INFINITY;
-        }
-        float bm = s[0];
+            for (int st = 0; st < NS; st++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[st], qh[st], s, 0, 0, 0);
+            // lane (j, hh) register r: query j, key k0 + 8 (r / 4) + 4 hh + r % 4
+            if (k0 + KB - 1 > p.index_pos + qb) {  // the block holds keys past some row
 #pragma unroll
-        for (int r = 1; r < 16; r++) bm = fmaxf(bm, s[r]);
-        bm = max_halves(bm);
-        const float sc = ldexpf(scq, e.x);
-        bm *= sc;
-        // the reference follows the max only where it lags by more than
-        // SLACK: the sums then need no rescaling in most blocks
-        const float mnew = bm > mrun + SLACK ? bm : mrun;
-        const float msafe = mnew == -INFINITY ? 0.0f : mnew;  // a block wholly past this query
-        const float scale = __builtin_amdgcn_exp2f(mrun - msafe);
-        float x[16], sum = 0.0f;
+                for (int r = 0; r < 16; r++)
+                    if (k0 + 8 * (r >> 2) + 4 * hh + (r & 3) > qpos) s[r] = -INFINITY;
+            }
+            float bm = s[0];
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], sc, -msafe));
-            sum += x[r];
-        }
-        lrun = __builtin_fmaf(lrun, scale, sum_halves(sum));
-        mrun = mnew;
+            for (int r = 1; r < 16; r++) bm = fmaxf(bm, s[r]);
+            bm = max_halves(bm);
+            const float sc = ldexpf(scq, e.x);
+            bm *= sc;
+            // the reference follows the max only where it lags by more than
+            // SLACK: the sums then need no rescaling in most blocks
+            const float mnew = bm > mrun + SLACK ? bm : mrun;
+            const float msafe = mnew == -INFINITY ? 0.0f : mnew;  // a block wholly past this query
+            const float scale = __builtin_amdgcn_exp2f(mrun - msafe);
+            float x[16], sum = 0.0f;
 #pragma unroll
-        for (int st = 0; st < 2; st++) split_p(x + 8 * st, ph[st], pl[st]);
-        const float os = ldexpf(scale, eo - e.y);
-        eo = e.y;
-        if (__any(os != 1.0f)) {
+            for (int r = 0; r < 16; r++) {
+                x[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], sc, -msafe));
+                sum += x[r];
+            }
+            lrun = __builtin_fmaf(lrun, scale, sum_halves(sum));
+            mrun = mnew;
 #pragma unroll
-            for (int b = 0; b < NB; b++)
+            for (int st = 0; st < 2; st++) split_p(x + 8 * st, ph[st], pl[st]);
+            const float os = ldexpf(scale, eo - e.y);
+            eo = e.y;
+            if (__any(os != 1.0f)) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[b][r] *= os;
-        }
-    };
-    auto values = [&](const uint8_t *vst) {
-        v8h vh[2], vl[2];
-        auto load = [&](int i) {  // fragment i: [2][NB]
-            vl[i & 1] = *(const v8h *)(vst + 64 * HD + (i * 64 + lane) * 16);
-            vh[i & 1] = *(const v8h *)(vst + (i * 64 + lane) * 16);
+                for (int b = 0; b < NB; b++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[b][r] *= os;
+            }
         };
-        load(0);
+        auto values = [&](const uint8_t *vst) {
+            v8h vh[2], vl[2];
+            auto load = [&](int i) {  // fragment i: [2][NB]
+                vl[i & 1] = *(const v8h *)(vst + 64 * HD + (i * 64 + lane) * 16);
+                vh[i & 1] = *(const v8h *)(vst + (i * 64 + lane) * 16);
+            };
+            load(0);
 #pragma unroll
-        for (int i = 0; i < 2 * NB; i++) {
-            const int st = i / NB, b = i % NB;
-            if (i + 1 < 2 * NB) load(i + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[i & 1], ph[st], o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i & 1], pl[st], o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i & 1], ph[st], o[b], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    auto live = [&](int it) {  // uniform over the wavefront
-        const int blk = it * KG + kg;
-        return blk < nkb && blk * KB <= p.index_pos + qb + KB - 1;
-    };
-    if constexpr (DB) {
-        for (int it = 0; it < nit; it++) {
-            wait_vmcnt<0>();  // this block's K and V
-            lds_barrier();    // everyone's, and everyone has read the last block's
-            next_exps(it);
-            issue(it + 1, 0);
-            issue(it + 1, BLK / 2);
-            const uint8_t *const base = lds + (kg * 2 + (it & 1)) * BLK;
-            if (live(it)) {
-                scores(it * KG + kg, base);
-                values(base + BLK / 2);
+            for (int i = 0; i < 2 * NB; i++) {
+                const int st = i / NB, b = i % NB;
+                if (i + 1 < 2 * NB) load(i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[i & 1], ph[st], o[b], 0, 0, 0);
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i & 1], pl[st], o[b], 0, 0, 0);
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i & 1], ph[st], o[b], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        auto live = [&](int it) {  // uniform over the wavefront
+            const int blk = it * KG + kg;
+            return blk < nkb && blk * KB <= p.index_pos + qb + KB - 1;
+        };
+        if constexpr (DB) {
+            for (int it = 0; it < nit; it++) {
+                wait_vmcnt<0>();  // this block's K and V
+                lds_barrier();    // everyone's, and everyone has read the last block's
+                next_exps(it);
+                issue(it + 1, 0);
+                issue(it + 1, BLK / 2);
+                const uint8_t *const base = lds + (kg * 2 + (it & 1)) * BLK;
+                if (live(it)) {
+                    scores(it * KG + kg, base);
+                    values(base + BLK / 2);
+                }
+            }
+        } else {
+            for (int it = 0; it < nit; it++) {
+                wait_vmcnt<0>();  // this block's K
+                lds_barrier();    // everyone's, and everyone has read the last block's V
+                next_exps(it);
+                issue(it, BLK / 2);
+                if (live(it)) scores(it * KG + kg, lds + kg * BLK);
+                wait_vmcnt<0>();  // this block's V
+                lds_barrier();    // everyone's, and everyone has read K
+                issue(it + 1, 0);
+                if (live(it)) values(lds + kg * BLK + BLK / 2);
             }
         }
-    } else {
-        for (int it = 0; it < nit; it++) {
-            wait_vmcnt<0>();  // this block's K
-            lds_barrier();    // everyone's, and everyone has read the last block's V
-            next_exps(it);
-            issue(it, BLK / 2);
-            if (live(it)) scores(it * KG + kg, lds + kg * BLK);
-            wait_vmcnt<0>();  // this block's V
-            lds_barrier();    // everyone's, and everyone has read K
-            issue(it + 1, 0);
-            if (live(it)) values(lds + kg * BLK + BLK / 2);
-        }
+        wait_vmcnt<0>();  // (copies past the last block write zeros)
     }
-    wait_vmcnt<0>();  // (copies past the last block write zeros)
 
     // combine the KG key ranges: M = max m, out = sum e^(m - M) o / sum e^(m - M) l
 #pragma unroll

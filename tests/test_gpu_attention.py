@@ -489,7 +489,10 @@ def test_prefill_one_large_key(env, hd, where, exp):
     for rows in (slice(0, 31), slice(31, m)):
         c = clear[rows]
         assert c.mean() > 0.7
-        assert a[rows][c].max() <= 1.5 * b[rows][c].max(), (rows, a[rows][c].max(), b[rows][c].max())
+        # (the largest error of a few hundred rows differs by half between two orders of
+        # the same f32 sums; its bound is test_prefill_split_operands')
+        rms = [np.sqrt((e[rows][c] ** 2).mean()) for e in (a, b)]
+        assert rms[0] <= 1.2 * rms[1] and a[rows][c].max() <= 1e-5, (rows, rms, a[rows][c].max())
 
 
 # The range inside a block of V: one key far above the others of its block, at each
