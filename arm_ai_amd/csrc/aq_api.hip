@@ -557,8 +557,8 @@ int aq_qmatmul_f32_device_noalloc(aq_ctx *ctx, const aq_qweight *w, const float 
     if ((rc = use_device(ctx->device))) return rc;
     const bool gemm = use_gemm(w, m);
     CallLayout L = call_layout(w, m, false, false, gemm);
-    // a K-quant GEMM splits K only as far as its partials fit
-    const size_t need = gemm && w->glayout.type != TYPE_Q8_0 ? L.ws : L.total;
+    // a GEMM splits K only as far as its partials fit
+    const size_t need = gemm ? L.ws : L.total;
     if (need > FIXED_SCRATCH_BYTES)
         return fail(AQ_ERR_SHAPE, "m=%lld needs %zu bytes of scratch, more than the fixed %zu; use aq_qmatmul_f32_device",
                     (long long)m, need, FIXED_SCRATCH_BYTES);

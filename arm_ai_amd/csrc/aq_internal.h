@@ -228,7 +228,7 @@ hipError_t launch_mmv(const WLayout &w, int64_t n, int64_t k, const ActPlanes &a
 // Prefill GEMM on MFMA (m > 8).  Returns hipErrorNotSupported for shapes it
 // does not take; the caller then uses launch_matvec.  ws: gemm_workspace_bytes
 // of scratch (split-K partials, summed by a second launch on the stream); with
-// less, the K-quant GEMMs split less.
+// less, the GEMM splits less.
 constexpr int GEMM_MAX_TILES = 1 << 20;
 hipError_t launch_gemm(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, int64_t m, float *y, int32_t *S,
                        int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s);

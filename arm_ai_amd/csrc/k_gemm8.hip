@@ -381,6 +381,24 @@ Gemm8Plan gemm8_plan(int64_t m, int64_t n, int64_t k) {
     return best;
 }
 
+// The same with the partials held to `room` bytes: fewer splits.
+Gemm8Plan gemm8_plan_in(int64_t m, int64_t n, int64_t k, size_t room) {
+    Gemm8Plan g = gemm8_plan(m, n, k);
+    if (g.ws > room) {
+        const int ng = (int)((k / QK8_0 + 7) / 8), most = std::max(1, (int)(room / ((size_t)m * n * 4)));
+        g.splits = std::min(g.splits, most);
+        g.kgs = (ng + g.splits - 1) / g.splits;
+        g.splits = (ng + g.kgs - 1) / g.kgs;
+        g.ws = g.splits > 1 ? (size_t)g.splits * m * n * 4 : 0;
+        if (g.form && g.kgs > Q8_FEW_MAX_GROUPS) {
+            g.form = 0;
+            g.ntm = (int)((m + COST[0].rows - 1) / COST[0].rows);
+            g.ntn = (int)((n + COST[0].cols - 1) / COST[0].cols);
+        }
+    }
+    return g;
+}
+
 // Rows per launch: the copies address the activation quants with 32-bit
 // offsets (rows * k < 2^31); longer inputs run as several launches.
 int64_t gemm8_chunk_rows(int64_t m, int64_t k) {
@@ -413,13 +431,12 @@ hipError_t launch_gemm8(const WLayout &w, int64_t n, int64_t k, const ActPlanes 
     const int64_t nb = k / QK8_0;
     for (int64_t r0 = 0; r0 < m; r0 += mc) {
         const int64_t mm = std::min(mc, m - r0);
-        Gemm8Plan g = gemm8_plan(mm, n, k);
+        Gemm8Plan g = gemm8_plan_in(mm, n, k, ws ? ws_bytes : 0);
         if (S) {  // the dump's form: few rows, split as far as d in LDS asks
             g = {1, (int)((mm + 31) / 32), (int)((n + 31) / 32), (w.ng + Q8_FEW_MAX_GROUPS - 1) / Q8_FEW_MAX_GROUPS, 0, 0};
             g.kgs = (w.ng + g.splits - 1) / g.splits;
         }
         if ((int64_t)g.ntm * g.ntn > GEMM_MAX_TILES) return hipErrorNotSupported;
-        if (g.ws && (!ws || ws_bytes < g.ws)) return hipErrorInvalidValue;
         Gemm8Params p;
         p.w = w.slab;
         p.rb_stride = w.rb_stride;

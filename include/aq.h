@@ -115,10 +115,12 @@ int aq_qmatmul_f32_device(aq_ctx *ctx, const aq_qweight *w, const float *d_lhs, 
  * such as code under HIP graph capture or a serving loop that forbids
  * hipMalloc.  The quantised activation and the prefill GEMM's workspace live
  * in a fixed array of aq_fixed_scratch_bytes() (32 MiB) per GPU, held until
- * the process ends; a call whose m, k and n need more returns AQ_ERR_SHAPE
- * (aq_qmatmul_f32_device has no such limit).  Every call on one GPU shares
+ * the process ends; a call that needs more returns AQ_ERR_SHAPE
+ * (aq_qmatmul_f32_device has no such limit): for a GEMM one whose quantised
+ * activation does, as the GEMM splits K only as far as its partial sums fit.  Every call on one GPU shares
  * that array, so calls that overlap on one GPU (two streams, two threads)
- * race: serialise them.  Same results as aq_qmatmul_f32_device. */
+ * race: serialise them.  Same results as aq_qmatmul_f32_device, in another
+ * order of the f32 sums where the GEMM splits less. */
 int aq_qmatmul_f32_device_noalloc(aq_ctx *ctx, const aq_qweight *w, const float *d_lhs, int64_t m, int64_t k,
                                   float *d_dst);
 size_t aq_fixed_scratch_bytes(void);

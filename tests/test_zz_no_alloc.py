@@ -51,6 +51,25 @@ def test_noalloc_matches_the_allocating_entry(ctx, wtype, n, k, ms):
     mm.free()
 
 
+# K splits whose partial sums would pass the array: the GEMM splits less instead
+# (646 x 12288 x 14336: 30 MB of activation planes and two splits of 30 MB), so the
+# sums come in another order
+@pytest.mark.parametrize("wtype,m,n,k", [(S.TYPE_Q8_0, 555, 1024, 8192), (S.TYPE_Q4_K, 555, 1024, 8192),
+                                         (S.TYPE_Q8_0, 646, 12288, 14336)])
+def test_noalloc_splits_what_fits(ctx, wtype, m, n, k):
+    rng = np.random.default_rng(n)
+    W = S.make_weight_unit(wtype, min(n, 1024), k, rng=rng)
+    blocks = np.tile(W.blocks.reshape(-1), -(-n // 1024))
+    mm = A.QMatMul.from_qtensor(A.QTensor(wtype, (n, k), blocks), ctx)
+    x = np.tile(S.make_activation(37, k, seed=m), (18, 1))[:m]
+    ya, yb = _both(ctx, mm, x)
+    assert float(np.abs(ya - yb).max()) <= 1e-5 * float(np.abs(ya).max())
+    r = O.matmul(wtype, x[:37], W.blocks, min(n, 1024), k)
+    tol = 1e-4 if k >= 14336 else 1e-5
+    assert float(np.abs(yb[:37, :1024] - r).max()) <= tol * float(np.abs(r).max())
+    mm.free()
+
+
 def test_noalloc_rejects_shapes_beyond_its_scratch(ctx):
     L = _lib.load()
     cap = L.aq_fixed_scratch_bytes()
