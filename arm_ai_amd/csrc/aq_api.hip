@@ -628,12 +628,12 @@ int aq_qmatmul2_preq_device(aq_ctx *ctx, const aq_qweight *w1, const aq_qweight 
     if ((uintptr_t)d_act & 255) return fail(AQ_ERR_INVALID_ARG, "activation buffer must be 256-byte aligned");
     if ((rc = use_device(ctx->device))) return rc;
     hipError_t e = hipErrorNotSupported;
-    if (use_gemm(w1, m) && use_gemm(w2, m)) {
-        const size_t ws = gemm_pair_workspace_bytes(m, w2->n, k);  // the second GEMM's split-K partials
-        if ((rc = ensure_scratch(ctx, ws))) return rc;
+    const size_t ws = use_gemm(w1, m) && use_gemm(w2, m)  // the second GEMM's split-K partials
+                          ? gemm_pair_workspace_bytes(w1->glayout.type, w2->glayout.type, m, w1->n, w2->n, k)
+                          : (size_t)-1;
+    if (ws != (size_t)-1 && ensure_scratch(ctx, ws) == AQ_OK)  // (without, the two calls)
         e = launch_gemm_pair(w1->glayout, w1->n, d_y1, w2->glayout, w2->n, d_y2, k, act_planes((void *)d_act, m, k), m,
                              ctx->scratch, ws, ctx->stream);
-    }
     if (e == hipSuccess) return AQ_OK;
     if (e != hipErrorNotSupported) return fail(AQ_ERR_HIP, "paired gemm: %s", hipGetErrorString(e));
     if ((rc = aq_qmatmul_preq_device(ctx, w1, d_act, m, k, d_y1))) return rc;

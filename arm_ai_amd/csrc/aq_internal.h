@@ -245,8 +245,8 @@ hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLay
 size_t gemm_workspace_bytes(int type, int64_t m, int64_t n, int64_t k);
 // The fewest rows for which launch_gemm is the faster path.
 int gemm_min_rows(int type, int64_t k);
-// Workspace that lets launch_gemm_pair split its second weight as far as it would.
-size_t gemm_pair_workspace_bytes(int64_t m, int64_t n2, int64_t k);
+// Workspace of launch_gemm_pair, or (size_t)-1 where it does not take the pair.
+size_t gemm_pair_workspace_bytes(int type1, int type2, int64_t m, int64_t n1, int64_t n2, int64_t k);
 // y[e] = part[0][e] + part[1][e] + ... of `total` elements, in split order.
 hipError_t launch_reduce(const float *part, float *y, int64_t total, int splits, hipStream_t s);
 // The Q8_0 GEMM on int8 MFMA (k_gemm8.hip), reached through launch_gemm /

@@ -226,37 +226,46 @@ hipError_t launch_gemm(const WLayout &w, int64_t n, int64_t k, const ActPlanes &
     return hipSuccess;
 }
 
-hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLayout &w2, int64_t n2, float *y2,
-                            int64_t k, const ActPlanes &x, int64_t m, void *ws, size_t ws_bytes, hipStream_t s) {
-    if (w1.type != TYPE_Q4_K || (w2.type != TYPE_Q6_K && w2.type != TYPE_Q5_K)) return hipErrorNotSupported;
-    if (!w1.slab || !w2.slab || (w2.type == TYPE_Q6_K && !w2.d) || !y1 || !y2 || !x.q16 || !x.d || !x.bsum16)
-        return hipErrorInvalidValue;
-    if (m <= 0 || n1 <= 0 || n2 <= 0 || k <= 0 || k % QK_K || m > 0x7fffffff || n1 > 0x7fffffff ||
-        n2 > 0x7fffffff || k > (1 << 24) || w1.ng != k / QK_K || w2.ng != k / QK_K)
-        return hipErrorInvalidValue;
-    if ((int64_t)16 * w1.rb_stride >= ((int64_t)1 << 31) || (int64_t)16 * w2.rb_stride >= ((int64_t)1 << 31))
-        return hipErrorNotSupported;
-    if (kq_chunk_rows(m, k) < m) return hipErrorNotSupported;
-    // Both as 64 x 128 tiles, the first weight unsplit, the second split
-    // until its steps are at most half as many, and together no more
-    // workgroups than the CUs hold at once (two each).
-    const int ng = w1.ng;
+// Both weights as 64 x 128 tiles, the first unsplit, the second split until its
+// steps are at most half as many, and together no more workgroups than the CUs
+// hold at once (two each); false where the two do not run as one launch.
+static bool pair_plan(int type1, int type2, int64_t m, int64_t n1, int64_t n2, int64_t k, Plan &g1, Plan &g2) {
+    if (type1 != TYPE_Q4_K || (type2 != TYPE_Q6_K && type2 != TYPE_Q5_K)) return false;
+    if (m <= 0 || n1 <= 0 || n2 <= 0 || k <= 0 || k % QK_K || m > 0x7fffffff || n1 > 0x7fffffff || n2 > 0x7fffffff ||
+        k > (1 << 24) || kq_chunk_rows(m, k) < m)
+        return false;
+    const int ng = (int)(k / QK_K);
     const int64_t ntm = (m + KQ_FORMS[1].rows - 1) / KQ_FORMS[1].rows;
     const int64_t t1 = ntm * ((n1 + 127) / 128), t2 = ntm * ((n2 + 127) / 128);
     int splits = 1;
     while (t1 + 2 * t2 * splits <= 512 && ng / (2 * splits) >= 2) splits *= 2;
-    if (t1 + t2 * splits > 512) return hipErrorNotSupported;
-    Plan g1{1, (int)ntm, (int)((n1 + 127) / 128), 1, ng, 0};
-    Plan g2{1, (int)ntm, (int)((n2 + 127) / 128), splits, (ng + splits - 1) / splits, 0};
-    g2.splits = (ng + g2.kbs - 1) / g2.kbs;
-    if (g2.splits > 1 && (!ws || ws_bytes < (size_t)g2.splits * m * n2 * 4)) return hipErrorNotSupported;
+    if (t1 + t2 * splits > 512) return false;
+    const int kbs = (ng + splits - 1) / splits, ns = (ng + kbs - 1) / kbs;
+    if (ns > 16) return false;
+    g1 = {1, (int)ntm, (int)((n1 + 127) / 128), 1, ng, 0};
+    g2 = {1, (int)ntm, (int)((n2 + 127) / 128), ns, kbs, ns > 1 ? (size_t)ns * m * n2 * 4 : 0};
+    return true;
+}
+
+size_t gemm_pair_workspace_bytes(int type1, int type2, int64_t m, int64_t n1, int64_t n2, int64_t k) {
+    Plan g1, g2;
+    return pair_plan(type1, type2, m, n1, n2, k, g1, g2) ? g2.ws : (size_t)-1;
+}
+
+hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLayout &w2, int64_t n2, float *y2,
+                            int64_t k, const ActPlanes &x, int64_t m, void *ws, size_t ws_bytes, hipStream_t s) {
+    Plan g1, g2;
+    if (!pair_plan(w1.type, w2.type, m, n1, n2, k, g1, g2) || g2.ws > (ws ? ws_bytes : 0)) return hipErrorNotSupported;
+    if (!w1.slab || !w2.slab || (w2.type == TYPE_Q6_K && !w2.d) || !y1 || !y2 || !x.q16 || !x.d || !x.bsum16 ||
+        w1.ng != k / QK_K || w2.ng != k / QK_K)
+        return hipErrorInvalidValue;
+    if ((int64_t)16 * w1.rb_stride >= ((int64_t)1 << 31) || (int64_t)16 * w2.rb_stride >= ((int64_t)1 << 31))
+        return hipErrorNotSupported;
     const KqParams p = kq_params(w1, n1, k, x, 0, m, g1, y1, nullptr, nullptr);
     const KqParams q = kq_params(w2, n2, k, x, 0, m, g2, g2.splits > 1 ? (float *)ws : y2, nullptr, nullptr);
     hipError_t e = launch_kq_pair(p, q, w2.type, s);
     if (e == hipSuccess && g2.splits > 1) e = launch_reduce((const float *)ws, y2, m * n2, g2.splits, s);
     return e;
 }
-
-size_t gemm_pair_workspace_bytes(int64_t m, int64_t n2, int64_t k) { return (size_t)std::min<int64_t>(k / QK_K, 16) * m * n2 * 4; }
 
 }  // namespace aq

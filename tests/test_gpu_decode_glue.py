@@ -703,6 +703,40 @@ def test_qmatmul2_preq_equals_two_calls(env, t1, t2, n1, n2, k, m):
     mm2.free()
 
 
+def test_qmatmul2_preq_keeps_no_scratch_for_a_declined_pair():
+    """A prompt whose two weights have more tiles than one launch takes runs the
+    two calls, and the context's scratch does not grow for the launch that did
+    not run (2048 rows: the partial sums of a split w2 would be 512 MiB)."""
+    import torch
+
+    import arm_ai_amd as A
+    from arm_ai_amd import _lib as lib
+    from arm_ai_amd import synth as S
+
+    L = lib.load()
+    n, k, m = 4096, 4096, 2048
+    with A.Context(0) as ctx:
+        mms = [A.QMatMul.from_qtensor(A.QTensor(t, (n, k), S.make_weight_unit(t, n, k, seed=t).blocks), ctx) for t in (12, 14)]
+        g = torch.Generator(device="cuda:0")
+        g.manual_seed(1)
+        x = torch.randn((m, k), generator=g, device="cuda:0")
+        act = _act(torch, lib, m, k)
+        y = [torch.empty((m, n), device="cuda:0") for _ in range(4)]
+        torch.cuda.synchronize()
+        lib.check(L.aq_quantize_act_device(ctx.handle, 15, x.data_ptr(), m, k, act.data_ptr()))
+        for mm, out in zip(mms, y):
+            lib.check(L.aq_qmatmul_preq_device(ctx.handle, mm.handle, act.data_ptr(), m, k, out.data_ptr()))
+        ctx.synchronize()
+        free = torch.cuda.mem_get_info(0)[0]
+        lib.check(L.aq_qmatmul2_preq_device(ctx.handle, mms[0].handle, mms[1].handle, act.data_ptr(), m, k, y[2].data_ptr(),
+                                            y[3].data_ptr()))
+        ctx.synchronize()
+        assert free - torch.cuda.mem_get_info(0)[0] < 16 << 20
+        assert torch.equal(y[2], y[0]) and torch.equal(y[3], y[1])
+        for mm in mms:
+            mm.free()
+
+
 def test_prompt_glue_act_errors(env):
     torch, lib, ctx = env
     L = lib.load()
