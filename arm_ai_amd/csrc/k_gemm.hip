@@ -68,6 +68,7 @@ struct FormCost {
 constexpr FormCost COST[] = {{1.4f, 0.84f, 2, 1},  {1.7f, 1.27f, 3, 1}, {4.3f, 4.3f, 1, 1},
                              {2.85f, 2.26f, 2, 1}, {1.3f, 1.4f, 3, 4},   {2.5f, 3.7f, 1, 8}};
 constexpr int NFORMS = 6;
+constexpr int MAX_SPLITS = 16;
 // The time of a step against Q4_K's.  A form of 32 rows builds the weight
 // operands for one row tile only, which costs most where they are two digits
 // (Q6_K): 512 x 2048 x 5632 takes 49.3 us in 32 x 128 tiles, 40.7 in 64 x 128 with
@@ -81,7 +82,7 @@ float step_weight(int type, int form) {
 Plan kq_plan(int type, int64_t m, int64_t n, int64_t k) {
     const int ng = (int)(k / QK_K);
     // up to 8 rows no split: those calls never needed a workspace
-    const int most_splits = m <= 8 ? 1 : 16;
+    const int most_splits = m <= 8 ? 1 : MAX_SPLITS;
     Plan best{};
     float best_us = 0.0f;
     for (int form = 0; form < NFORMS; form++) {
@@ -238,10 +239,9 @@ static bool pair_plan(int type1, int type2, int64_t m, int64_t n1, int64_t n2, i
     const int64_t ntm = (m + KQ_FORMS[1].rows - 1) / KQ_FORMS[1].rows;
     const int64_t t1 = ntm * ((n1 + 127) / 128), t2 = ntm * ((n2 + 127) / 128);
     int splits = 1;
-    while (t1 + 2 * t2 * splits <= 512 && ng / (2 * splits) >= 2) splits *= 2;
+    while (splits < MAX_SPLITS && t1 + 2 * t2 * splits <= 512 && ng / (2 * splits) >= 2) splits *= 2;
     if (t1 + t2 * splits > 512) return false;
     const int kbs = (ng + splits - 1) / splits, ns = (ng + kbs - 1) / kbs;
-    if (ns > 16) return false;
     g1 = {1, (int)ntm, (int)((n1 + 127) / 128), 1, ng, 0};
     g2 = {1, (int)ntm, (int)((n2 + 127) / 128), ns, kbs, ns > 1 ? (size_t)ns * m * n2 * 4 : 0};
     return true;

@@ -703,6 +703,37 @@ def test_qmatmul2_preq_equals_two_calls(env, t1, t2, n1, n2, k, m):
     mm2.free()
 
 
+def test_qmatmul2_preq_of_long_rows(env):
+    """Few tiles and 128 super-blocks: the pair runs with its second weight in 16
+    splits (its workspace of 16 partial sums shows that it is not declined).
+    Two orders of 128 f32 terms differ by at most 128 * 2^-24 of the largest sum."""
+    import arm_ai_amd as A
+    from arm_ai_amd import synth as S
+
+    torch, lib, ctx = env
+    L = lib.load()
+    n1, n2, k, m = 256, 128, 32768, 20
+    ws = getattr(L, "_ZN2aq25gemm_pair_workspace_bytesEiillll")  # (internal: k_gemm.hip)
+    ws.restype, ws.argtypes = ctypes.c_size_t, [ctypes.c_int] * 2 + [ctypes.c_int64] * 4
+    assert ws(12, 14, m, n1, n2, k) == 16 * m * n2 * 4
+    mms = [A.QMatMul.from_qtensor(A.QTensor(t, (n, k), S.make_weight_unit(t, n, k, seed=t).blocks), ctx)
+           for t, n in ((12, n1), (14, n2))]
+    dx = _dev(torch, np.random.default_rng(m).standard_normal((m, k)).astype(np.float32))
+    act = _act(torch, lib, m, k)
+    y = [torch.empty((m, n), device="cuda:0") for n in (n1, n2, n1, n2)]
+    torch.cuda.synchronize()
+    lib.check(L.aq_quantize_act_device(ctx.handle, 15, dx.data_ptr(), m, k, act.data_ptr()))
+    lib.check(L.aq_qmatmul2_preq_device(ctx.handle, mms[0].handle, mms[1].handle, act.data_ptr(), m, k, y[0].data_ptr(),
+                                        y[1].data_ptr()))
+    for mm, out in zip(mms, y[2:]):
+        lib.check(L.aq_qmatmul_preq_device(ctx.handle, mm.handle, act.data_ptr(), m, k, out.data_ptr()))
+    ctx.synchronize()
+    for got, want in ((y[0], y[2]), (y[1], y[3])):
+        assert float((got - want).abs().max()) <= 128 * 2.0 ** -24 * float(want.abs().max())
+    for mm in mms:
+        mm.free()
+
+
 def test_qmatmul2_preq_keeps_no_scratch_for_a_declined_pair():
     """A prompt whose two weights have more tiles than one launch takes runs the
     two calls, and the context's scratch does not grow for the launch that did
