@@ -239,7 +239,7 @@ CallLayout call_layout(const aq_qweight *w, int64_t m, bool host_io, bool dump, 
 }
 
 bool use_gemm(const aq_qweight *w, int64_t m) {
-    return m >= gemm_min_rows(w->glayout.type, w->k) && gemm_workspace_bytes(w->glayout.type, m, w->n, w->k) != (size_t)-1;
+    return m >= gemm_min_rows(w->type, w->n, w->k) && gemm_workspace_bytes(w->glayout.type, m, w->n, w->k) != (size_t)-1;
 }
 // 2 or more rows of Q4_K / Q6_K without a GEMM: quantizer kernel, then the
 // matrix-core matvec

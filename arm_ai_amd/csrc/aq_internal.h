@@ -243,8 +243,8 @@ hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLay
 // Workspace bytes launch_gemm needs for this shape, or (size_t)-1 if the
 // weight type / shape has no GEMM (the matvec then serves m > 8 too).
 size_t gemm_workspace_bytes(int type, int64_t m, int64_t n, int64_t k);
-// The fewest rows for which launch_gemm is the faster path.
-int gemm_min_rows(int type, int64_t k);
+// The fewest rows for which launch_gemm is the faster path (type: the weight's own).
+int gemm_min_rows(int type, int64_t n, int64_t k);
 // Workspace of launch_gemm_pair, or (size_t)-1 where it does not take the pair.
 size_t gemm_pair_workspace_bytes(int type1, int type2, int64_t m, int64_t n1, int64_t n2, int64_t k);
 // y[e] = part[0][e] + part[1][e] + ... of `total` elements, in split order.
