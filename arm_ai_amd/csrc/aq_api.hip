@@ -259,8 +259,8 @@ int check_mm(aq_ctx *ctx, const aq_qweight *w, int64_t m, int64_t k) {
 // The matmul of d_x [m][k] into d_y on ctx->stream.  Rows enough for a GEMM
 // (gemm_min_rows): the quantizer kernel writes the activation planes at `act`, then
 // the GEMM.  Other m >= 2 of Q4_K / Q6_K: the quantizer, then the
-// matrix-core matvec (passes of 8 rows).  Otherwise (m = 1, Q8_0): one matvec
-// launch that quantises d_x itself.
+// matrix-core matvec (passes of 8 rows).  Otherwise (one row, or fewer of another
+// type than the GEMM takes): one matvec launch that quantises d_x itself.
 int run_matmul(aq_ctx *ctx, const aq_qweight *w, const float *d_x, int64_t m, float *d_y, void *act, int32_t *dS,
                int32_t *dSmin, void *ws, size_t ws_bytes) {
     hipError_t e;

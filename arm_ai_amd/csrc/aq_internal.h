@@ -89,7 +89,8 @@ inline int groups_of(int type, int64_t k) {
 //   q16   m * k       the qs as f16 bits, the activation operand of the
 //                     K-quant GEMMs, in the order in which their MFMAs read
 //                     it (q16_at); written by the Q8_K quantizers when the
-//                     pointer is set (paths that feed no such GEMM clear it)
+//                     pointer is set (paths that feed no such GEMM clear it).
+//                     The Q8_0 quantizer keeps its GEMM's planes there (q8_at)
 struct ActPlanes {
     int8_t *qs;
     float *d;
@@ -225,7 +226,7 @@ int mmv_max_k();
 size_t mmv_workspace_bytes(int type, int64_t n, int64_t k);
 hipError_t launch_mmv(const WLayout &w, int64_t n, int64_t k, const ActPlanes &act, int64_t m, float *y, int32_t *S,
                       int32_t *Smin, void *ws, size_t ws_bytes, hipStream_t s);
-// Prefill GEMM on MFMA (m > 8).  Returns hipErrorNotSupported for shapes it
+// Prefill GEMM on MFMA.  Returns hipErrorNotSupported for shapes it
 // does not take; the caller then uses launch_matvec.  ws: gemm_workspace_bytes
 // of scratch (split-K partials, summed by a second launch on the stream); with
 // less, the GEMM splits less.
@@ -241,7 +242,7 @@ hipError_t launch_gemm(const WLayout &w, int64_t n, int64_t k, const ActPlanes &
 hipError_t launch_gemm_pair(const WLayout &w1, int64_t n1, float *y1, const WLayout &w2, int64_t n2, float *y2,
                             int64_t k, const ActPlanes &x, int64_t m, void *ws, size_t ws_bytes, hipStream_t s);
 // Workspace bytes launch_gemm needs for this shape, or (size_t)-1 if the
-// weight type / shape has no GEMM (the matvec then serves m > 8 too).
+// weight type / shape has no GEMM (the matvec then serves every m).
 size_t gemm_workspace_bytes(int type, int64_t m, int64_t n, int64_t k);
 // The fewest rows for which launch_gemm is the faster path (type: the weight's own).
 int gemm_min_rows(int type, int64_t n, int64_t k);

@@ -1,6 +1,6 @@
-// gemm_kq.h -- the prefill GEMM (m > 8) of the K-quant weights (Q4_K, Q5_K,
-// Q6_K, Q2_K, Q3_K) on the f16 matrix cores, gfx950: its kernel template and
-// parameters.  k_gemm.hip holds the launch plan; one small .hip file per
+// gemm_kq.h -- the prefill GEMM (from gemm_min_rows rows) of the K-quant weights
+// (Q4_K, Q5_K, Q6_K, Q2_K, Q3_K) on the f16 matrix cores, gfx950: its kernel
+// template and parameters.  k_gemm.hip holds the launch plan; one small .hip file per
 // weight type instantiates the template.
 //
 // Replaces the M-row loop of candle-core 0.8.4 k_quants::matmul<T> at
@@ -21,9 +21,13 @@
 //         the scale is split, sc = 16 sh + sl (sh in -8..7, sl in 0..15), into
 //         the operands sh (q - 32) and sl (q - 32) / 16 (at most 9 significant
 //         bits each) of one chain, which holds S / 16; one step stays exact
-// The output chains a whole super-block (an f32 sum that rounds only above 24
-// bits, which the sums of real files do not reach); the integer dump restarts
-// the chain where it could round and adds in int32.
+// The integer dump restarts the chain where it could round and adds in int32.  The
+// output chains a whole super-block: S is exact below 2^24 (Q6_K: while every
+// partial sum is), and rounded to 24 bits by each later step beyond, which the
+// sums of real files do not reach (normal activations: 2^21 on random weights).  Error
+// against 64 bits, 40 x 64 x 2048, Q4_K, Q5_K, Q6_K: normal activations 7.4e-8,
+// 7.2e-8, 6.5e-8 of the result; activations of one sign on the largest weights, S
+// up to 2^24.8, 2^25.8, 2^26.9: 6.9e-8, 6.4e-8, 5.0e-8.
 // Smin is one more f16 MFMA per tile and super-block (bsums <= 2048, mins <=
 // 63; every partial sum below 2^24).
 //

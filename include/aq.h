@@ -22,9 +22,10 @@
  *  - Weight type ids are GGUF/GGML dtype ids (Q4_0 = 2, Q5_0 = 6, Q8_0 = 8,
  *    Q2_K = 10, Q3_K = 11, Q4_K = 12, Q5_K = 13, Q6_K = 14).  Every type
  *    runs a matvec at m = 1 and small batches, and a prefill GEMM for more
- *    rows (m > 8; Q5_K, Q2_K and Q3_K m > 2, Q8_0, Q4_0 and Q5_0 m > 3; Q4_0
- *    and Q5_0 on an int8 copy that the upload expands into the Q8_0 layout,
- *    34 bytes per 32 weights beside their 18- or 22-byte decode tiles).
+ *    rows (Q4_K and Q6_K m > 8, the others from three to seven rows on by type
+ *    and shape; Q4_0 and Q5_0 on an int8 copy that the upload expands into the
+ *    Q8_0 layout, 34 bytes per 32 weights beside their 18- or 22-byte decode
+ *    tiles).
  *  - A weight is n rows (output features) by k columns (input features),
  *    row-major blocks, exactly candle's QTensor storage of shape (n, k).
  *  - Host-pointer entry points are synchronous at return.  Device-pointer
@@ -117,9 +118,9 @@ int aq_qmatmul_f32_device(aq_ctx *ctx, const aq_qweight *w, const float *d_lhs, 
  * in a fixed array of aq_fixed_scratch_bytes() (32 MiB) per GPU, held until
  * the process ends; a call that needs more returns AQ_ERR_SHAPE
  * (aq_qmatmul_f32_device has no such limit): for a GEMM one whose quantised
- * activation does, as the GEMM splits K only as far as its partial sums fit.  Every call on one GPU shares
- * that array, so calls that overlap on one GPU (two streams, two threads)
- * race: serialise them.  Same results as aq_qmatmul_f32_device, in another
+ * activation does, as the GEMM splits K only as far as its partial sums fit.
+ * Every call on one GPU shares that array, so calls that overlap on one GPU
+ * (two streams, two threads) race: serialise them.  Same results as aq_qmatmul_f32_device, in another
  * order of the f32 sums where the GEMM splits less. */
 int aq_qmatmul_f32_device_noalloc(aq_ctx *ctx, const aq_qweight *w, const float *d_lhs, int64_t m, int64_t k,
                                   float *d_dst);
@@ -305,7 +306,12 @@ int aq_llama_attn_decode(aq_ctx *ctx, const float *d_qk, const float *d_v, const
  * caches, then writes the causal softmax(q.k/sqrt(head_dim)).v over
  * positions 0 .. its own for every row and query head to d_out
  * [m][n_head*head_dim].  head_dim 64 or 128 (AQ_ERR_SHAPE otherwise); caches
- * and d_out 16-byte aligned. */
+ * and d_out 16-byte aligned.  Where (index_pos + m) * head_dim passes 20480 the
+ * call uses a workspace of the context, 8 * head_dim bytes per position and kv
+ * head, which grows in powers of two (the call then allocates, and waits for
+ * the stream before it frees the smaller one) and stays until the context is
+ * destroyed; calls on one context must not overlap.  Under capture, past 2 GiB
+ * or where it cannot be had, a kernel without it runs. */
 int aq_llama_attn_prefill(aq_ctx *ctx, const float *d_q, int64_t ldq, const float *d_k, int64_t ldk, const float *d_v,
                           int64_t ldv, const float *d_cos, const float *d_sin, int64_t index_pos, int64_t m,
                           float *d_kcache, float *d_vcache, int64_t n_head, int64_t n_kv, int64_t head_dim,
@@ -351,7 +357,7 @@ int aq_llama_swiglu_pairs(aq_ctx *ctx, const float *d_y, int64_t ld, int64_t m, 
  * (aq_llama_swiglu_pairs) with the result quantised to Q8_K in the same
  * launch, into the activation planes at d_act (aq_act_bytes(AQ_TYPE_Q8_K, m,
  * n or ffn) bytes, 256-byte aligned; the planes include the f16 copy of the
- * quants that the Q6_K / Q5_K GEMMs read) for aq_qmatmul_preq_device.  The
+ * quants that the K-quant GEMMs read) for aq_qmatmul_preq_device.  The
  * values are those of the unfused call followed by aq_quantize_act_device,
  * bit for bit; d_out, when non-null, receives the f32 values as well.  n is
  * a multiple of 256 up to 8192, ffn a multiple of 256 with m <= 65535 and ld

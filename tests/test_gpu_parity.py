@@ -120,7 +120,7 @@ def test_config4_llama3_lm_head_q6k(ctx):
     check_matmul(ctx, W, x, sums=False, cond=False)
 
 
-# ----------------------------------------------- prefill GEMM (int8 MFMA, m > 8)
+# ------------------------------------------ Q4_K prefill GEMM (f16 MFMA, m > 8)
 @pytest.mark.parametrize("n,k", [(5632, 2048), (2048, 5632)])
 def test_config3_prefill_gemm(ctx, n, k):
     W = S.make_weight(S.TYPE_Q4_K, n, k, seed=3)
@@ -304,7 +304,7 @@ def test_single_row_weight(ctx):
     check_matmul(ctx, W, x)
 
 
-# ------------------------------------ Q5_K (matvec m <= 8, f16 MFMA GEMM m > 8)
+# ---------------------------- Q5_K (matvec, f16 MFMA GEMM from three or four rows)
 @pytest.mark.parametrize("n,k,m", [(5632, 2048, 1), (2048, 5632, 1), (14336, 4096, 1), (4096, 14336, 8),
                                    (2048, 2048, 40)])
 def test_q5k_matvec(ctx, n, k, m):
@@ -377,7 +377,7 @@ def test_q4_0_matvec(ctx, n, k, m):
 
 @pytest.mark.parametrize("n,k,m", [(1024, 2048, 64), (300, 1056, 40), (2048, 96, 17)])
 def test_q4_0_prefill_gemm(ctx, n, k, m):
-    """m > 8: the Q8_0 GEMM on the upload's expanded copy (values q - 8 as
+    """The Q8_0 GEMM on the upload's expanded copy (values q - 8 as
     int8), including rows with padding blocks: block sums bit-exact."""
     W = S.make_weight(S.TYPE_Q4_0, n, k, seed=n + k + 9)
     x = S.make_activation(m, k, seed=m + k + 9)
@@ -397,12 +397,12 @@ def test_q4_0_extreme_values(ctx):
         check_matmul(ctx, W, x, cond=False)
 
 
-# ----------------------------- Q5_0 (matvec m <= 8, Q8_0 GEMM on a copy m > 8)
+# ---------------------- Q5_0 (matvec, Q8_0 GEMM on a copy from four or five rows)
 @pytest.mark.parametrize("n,k,m", [(14336, 4096, 1), (4096, 14336, 8), (300, 96, 3), (1024, 2048, 64),
                                    (300, 1056, 40)])
 def test_q5_0_matvec_and_gemm(ctx, n, k, m):
     """Llama-3 FFN shapes of a Q5_0 file, rows whose block count is not a
-    multiple of 8 (padding blocks), and m > 8 through the Q8_0 GEMM on the
+    multiple of 8 (padding blocks), and more rows through the Q8_0 GEMM on the
     upload's expanded copy (values q - 16): block sums bit-exact."""
     W = S.make_weight(S.TYPE_Q5_0, n, k, seed=n + k + 6)
     x = S.make_activation(m, k, seed=m + k + 6)
@@ -461,7 +461,7 @@ def test_q3k_extreme_values(ctx, qv, scv):
     check_matmul(ctx, W, x, cond=False)
 
 
-# ------------------------------------------ Q8_0 prefill GEMM (int8 MFMA, m > 8)
+# --------------------------- Q8_0 prefill GEMM (int8 MFMA, from four or five rows)
 @pytest.mark.parametrize("n,k,m", [(768, 2048, 256), (4096, 4096, 16)])
 def test_prefill_gemm_q8_0(ctx, n, k, m):
     """A 256-token prefill and a 16-row batch (four k-splits per tile):

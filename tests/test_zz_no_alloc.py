@@ -7,7 +7,7 @@ with a prefill-sized input (the GEMM path, which needs the scratch), the
 second with a smaller one (the array keeps the first call's contents, which
 must not leak into the second's result).  The kernels are the same, so the
 results must be identical to the bit.  Plus the one-row path, a Q6_K weight
-(the f16 GEMM, whose workspace also holds the f16 copy of the quants), and
+(the GEMM of two scale digits), and
 the size limit.
 """
 import numpy as np
@@ -33,8 +33,8 @@ def _both(ctx, mm, x):
 
 
 @pytest.mark.parametrize("wtype,n,k,ms", [
-    (S.TYPE_Q4_K, 2048, 5632, (64, 20, 1)),   # int8 GEMM, then a smaller GEMM, then the matvec
-    (S.TYPE_Q6_K, 2048, 2048, (96, 33)),      # f16 GEMM (quants copied to f16 in the scratch)
+    (S.TYPE_Q4_K, 2048, 5632, (64, 20, 1)),   # GEMM, then a smaller GEMM, then the matvec
+    (S.TYPE_Q6_K, 2048, 2048, (96, 33)),      # GEMM of two scale digits
     (S.TYPE_Q8_0, 1024, 4096, (48, 9)),       # Q8_0 GEMM (Q8_0 activation planes)
     (S.TYPE_Q4_K, 512, 14336, (8, 3)),        # batched matvec in K parts (the parts' sums in the scratch)
 ])
