@@ -495,6 +495,33 @@ def test_prefill_one_large_key(env, hd, where, exp):
         assert rms[0] <= 1.2 * rms[1] and a[rows][c].max() <= 1e-5, (rows, rms, a[rows][c].max())
 
 
+# The same key within the first of two pieces: the pieces (the second reads the key
+# from the cache) give what the whole prompt gives, to the bound of either.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("where", ["k", "v"])
+@pytest.mark.parametrize("exp", [0, 13, 24])
+def test_prefill_in_pieces(env, hd, where, exp):
+    torch, lib, ctx = env
+    n_head, n_kv, m, cut = 6, 2, 420, 257
+    rng = np.random.default_rng(hd + exp)
+    qk = rng.standard_normal((m, (n_head + n_kv) * hd)).astype(np.float32)
+    v = rng.standard_normal((m, n_kv * hd)).astype(np.float32)
+    (qk[:, n_head * hd:] if where == "k" else v)[201] *= 2.0 ** exp
+    cos, sin = _tables(hd, m)
+    z = np.zeros((n_kv, m, hd), np.float32)
+    whole, kw, vw = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, m, m, qk, v, z, z, cos, sin)
+    a, k1, v1 = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, 0, cut, m, qk[:cut], v[:cut], z, z, cos, sin)
+    b, k2, v2 = _prefill_call(torch, lib, ctx, n_head, n_kv, hd, cut, m - cut, m, qk[cut:], v[cut:], k1, v1, cos, sin)
+    assert np.array_equal(kw, k2) and np.array_equal(vw, v2)
+    s = _scores(qk, kw, cos, sin, n_head)
+    rest = np.where(np.arange(m) == 201, -np.inf, s).max(-1)
+    clear = np.ones((m, n_head), bool)
+    if where == "k":  # (a score of 2^exp against others: see above)
+        clear[201:] = (exp == 0) | (np.abs(s[201:, :, 201] - rest[201:]) > 30)
+    assert clear.mean() > 0.7
+    assert _row_errors(np.concatenate([a, b]), whole, m, n_head)[clear].max() <= 2e-5
+
+
 # The range inside a block of V: one key far above the others of its block, at each
 # place in it, and dims far below the others.  Each dim of the rows before that key
 # as exact as the f32 kernel has it (15: just past the range that the split takes,
