@@ -56,7 +56,7 @@ struct Plan {
 // holds, and the super-blocks of a step (the few-row forms' wavefronts take
 // one each).  A split adds the reduce launch and one write and read of its
 // partials.  Rows x columns x K, with the quantizer launch:
-//   512 x 14336 x 4096  128 x 256 tiles 78 us, 64 x 128 90 (71.4 the former on a faster box)
+//   512 x 14336 x 4096  128 x 256 tiles 78 us, 64 x 128 90 (71.4 the former on a faster card)
 //   512 x 5632 x 2048   64 x 128 28 us, 128 x 256 in two splits 33
 //   128 x 4096 x 4096   few rows 17.5 us, 64 x 128 in four splits 21.1
 //   512 x 2048 x 2048   32 x 128 tiles 18.9 us, 64 x 128 21.3, few rows 22.1

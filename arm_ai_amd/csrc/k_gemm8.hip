@@ -38,7 +38,7 @@
 // more fmas' time, and the error against 64 bits stays below that of the
 // 128 x 128 tiles before (8.5e-8 against 9.6e-8 at 333 x 4096 x 4096, where one
 // chain over K had 1.5e-7); 240 VGPRs, two wavefronts per SIMD.
-// 333 x 4096 x 4096: 40.6 us before, 32.6 now (40.9 and 33.2 on another box); 512 x
+// 333 x 4096 x 4096: 40.6 us before, 32.6 now (40.9 and 33.2 on another card); 512 x
 // 14336 x 4096: 131.6, 105.8; 512 x 5632 x 2048: 43.5, 31.6 (with the quantizer).
 // Few-row form (a tile of 32): the wavefronts of a workgroup share 32 columns
 // and take every fourth or eighth group each, with no stage and no barrier in

@@ -3,7 +3,7 @@
  * from compiled C, as the Rust NIF crate's `extern "C"` binding calls it,
  * checked against the CPU oracle (oracle/oracle.h, the restatement of
  * candle-core 0.8.4's k_quants).  Built by tests/c/Makefile with gcc; run by
- * tests/test_c_abi_program.py on a GPU box.  Test infrastructure: it links
+ * tests/test_c_abi_program.py on a GPU.  Test infrastructure: it links
  * the oracle as the checker.
  *
  * Checks, for Q4_K, Q6_K and Q8_0 weights built from seeded random bytes
