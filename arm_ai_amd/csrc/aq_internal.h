@@ -185,6 +185,8 @@ hipError_t launch_expand_q80(int type, const uint8_t *src, int64_t n, int64_t k,
 // S/Smin non-null selects the integer-dump variant ([m][n][blocks] int32).
 hipError_t launch_matvec(const WLayout &w, int64_t n, int64_t k, const float *x, const ActPlanes *act, int64_t m,
                          float *y, int32_t *S, int32_t *Smin, hipStream_t s);
+// The workgroups that share the rows of one of its passes (of several rows of x).
+int64_t matvec_workgroups(int type, int64_t n, int64_t k);
 // Batch-1 matvec with one weight row per lane (k_rowlane.hip) for Q4_K,
 // Q5_K, Q6_K, Q8_0, Q4_0, Q5_0, Q2_K and Q3_K weights of at least 256 rows, k
 // a multiple of 256 and <= 16384 (8192 for Q8_0); hipErrorNotSupported for

@@ -165,42 +165,42 @@ KqParams kq_params(const WLayout &w, int64_t n, int64_t k, const ActPlanes &x, i
 // Q5_K, Q2_K, Q3_K and the Q8_0 family have no matrix-core matvec, and the dot4
 // matvec's time grows with the rows: from three to seven rows on the GEMM's
 // few-row forms are faster, as far as they take the row length.  The line depends
-// on what the matvec reads (Q4_0 and Q5_0 are less than half and 0.65 of the copy
-// that the GEMM reads) and on whether the 32-column workgroups fit the CUs at once
-// (`wide`: past three a CU the few-row forms take a second turn; not felt in
-// short rows).  Matvec and GEMM, us:
+// on what the matvec reads (Q4_0 and Q5_0 are about half and 0.65 of the copy that
+// the GEMM reads), on whether its workgroups take a second turn on the CUs
+// (`turns`), and on the GEMM's workgroups of 32 columns: past one a CU beside a
+// matvec of one turn (`many`), past three a CU (`wide`); either is not felt in short
+// rows.  Matvec and GEMM, us (* turns):
 //   Q2_K  3 rows  14336 x 4096 15.0, 11.8   32000 x 2048 11.8, 13.0  128256 x 2048 32.1, 25.3
 //         4 rows  14336 x 4096 18.2, 11.8   32000 x 2048 14.2, 13.1   32000 x 4096 25.5, 20.8
-//   Q3_K  3 rows  14336 x 4096 16.3, 14.1   32000 x 2048 13.4, 14.8   32000 x 4096 23.4, 21.5
+//   Q3_K  3 rows  14336 x 4096 16.3, 14.1   32000 x 2048 13.4, 14.8   11008 x 2048  9.2,  9.8
 //         4 rows   4096 x 4096 13.8, 10.2   32000 x 2048 15.7, 14.9
-//   Q5_K  3 rows  14336 x 4096 14.5, 15.3   16384 x 1024  7.0,  8.2   4096 x 14336 24.3, 20.6
-//                 11008 x 4096 20.0, 15.4   49152 x 512  16.7,  9.8   32000 x 4096 26.3, 29.8
+//   Q5_K  3 rows  12288 x 4096 14.2, 15.4   16384 x 1024  7.0,  8.2   32000 x 4096 26.3, 29.8
+//                *20480 x 4096 24.5, 18.7  *24576 x 2048 14.8, 13.8   4096 x 14336 24.3, 20.6
 //         4 rows  14336 x 4096 16.9, 15.3   16384 x 1024  8.0,  8.1   32000 x 4096 30.6, 29.9
-//   Q8_0  4 rows  14336 x 4096 19.3, 18.2   16384 x 1024  8.5,  9.3   32000 x 4096 36.0, 38.2
+//   Q8_0  4 rows  14336 x 4096 19.3, 18.2   11008 x 2048 10.3, 11.6   32000 x 4096 36.0, 38.2
+//                *20480 x 4096 33.0, 23.4  *24576 x 1024 14.7, 10.8
 //         5 rows  14336 x 4096 22.1, 18.1   16384 x 1024  9.6,  9.2   32000 x 4096 44.0, 38.3
-//   Q5_0  4 rows  14336 x 4096 19.5, 18.3   16384 x 1024  9.4,  9.2   32000 x 4096 31.1, 38.6
-//         5 rows  14336 x 4096 22.8, 18.1   49152 x 576  26.5, 14.2   32000 x 4096 41.6, 38.6
-//   Q4_0  4 rows  14336 x 4096 17.4, 18.2    8192 x 2048  9.7,  9.6   32000 x 4096 26.8, 38.6
+//   Q5_0  4 rows  14336 x 4096 19.5, 18.3   11008 x 2048 10.8, 11.6   32000 x 4096 31.1, 38.6
+//         5 rows  14336 x 4096 22.8, 18.1  *49152 x 576  26.5, 14.2   32000 x 4096 41.6, 38.6
+//   Q4_0  4 rows  14336 x 4096 17.4, 18.2   11008 x 2048  9.9, 11.6   32000 x 4096 26.8, 38.6
+//                *20480 x 4096 25.6, 23.8  *24576 x 1024 12.2, 10.8   13824 x 5120 22.9, 21.0
 //         5 rows  14336 x 4096 21.0, 18.1   24576 x 2048 17.6, 15.4   32000 x 4096 32.2, 38.4
-//         6 rows  14336 x 4096 23.8, 18.1   49152 x 576  22.6, 14.2   32000 x 4096 36.5, 38.7
+//         6 rows  14336 x 4096 23.8, 18.1  *49152 x 576  22.6, 14.2   32000 x 4096 36.5, 38.7
 //         8 rows  14336 x 4096 29.6, 18.3                             32000 x 2048 25.0, 20.5
-// (Where the matvec's own grid ends unevenly, as at 11008, it keeps calls that the
-// GEMM would have faster; of 260 calls measured none is slower than its matvec by
-// more than 1.4 %.)
 // The matrix-core matvec keeps Q4_K and Q6_K up to its 8 rows (11.0 against 14.1 at
 // 8 x 14336 x 4096, 8.3 against 8.9 at 8 x 5632 x 2048).
 int gemm_min_rows(int type, int64_t n, int64_t k) {
     const bool wide = n > 3 * 256 * 32 && k >= 1024;
+    const bool turns = !wide && matvec_workgroups(type, n, k) > 256;
+    const bool many = !wide && !turns && n > 256 * 32 && k >= 1024;
     if (type == TYPE_Q8_0 || type == TYPE_Q4_0 || type == TYPE_Q5_0) {
         if (k > 256 * (int64_t)Q8_FEW_MAX_GROUPS) return 9;
-        const bool many = n > 8192 && k >= 1024;
-        if (type == TYPE_Q4_0) return wide ? 7 : many ? 5 : Q8_MIN_ROWS;
-        if (type == TYPE_Q5_0) return wide ? 5 : Q8_MIN_ROWS;
-        return wide || (many && k < 2048) ? 5 : Q8_MIN_ROWS;
+        if (type == TYPE_Q4_0) return wide ? 7 : many && k < 5120 ? 5 : Q8_MIN_ROWS;
+        return wide || (many && k <= 2048) ? 5 : Q8_MIN_ROWS;
     }
     if (k > QK_K * (int64_t)KQ_FEW_MAX_NG) return 9;
-    if (type == TYPE_Q2_K || type == TYPE_Q3_K) return wide && k < 4096 && n <= 65536 ? 4 : 3;
-    if (type == TYPE_Q5_K) return k > 8192 || (n > 8192 && k < 1024) ? 3 : 4;
+    if (type == TYPE_Q2_K || type == TYPE_Q3_K) return (wide && k < 4096 && n <= 65536) || (many && k > 1024 && k <= 2048) ? 4 : 3;
+    if (type == TYPE_Q5_K) return turns || k >= 5120 ? 3 : 4;
     return 9;
 }
 

@@ -984,6 +984,11 @@ hipError_t matvec_impl(const WLayout &w, int64_t n, int64_t k, const float *x, c
 
 }  // namespace
 
+int64_t matvec_workgroups(int type, int64_t n, int64_t k) {
+    const MvPlan P = mv_plan(n, groups_of(type, k));
+    return ((n + RB - 1) / RB + P.rbw - 1) / P.rbw;
+}
+
 hipError_t launch_matvec(const WLayout &w, int64_t n, int64_t k, const float *x, const ActPlanes *act, int64_t m,
                          float *y, int32_t *S, int32_t *Smin, hipStream_t s) {
     return matvec_impl(w, n, k, x, act, m, y, S, Smin, XfArgs{}, s);
